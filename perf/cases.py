@@ -215,6 +215,8 @@ def prepare(case, seed):
     inp = _inputs(case, seed)
     sd = _handle(case)
     st = {"case": case, "sd": sd, "inp": inp}
+    if case["op"] == "half":
+        sd.set_mixed_tolerance(1.5e-6)      # what the ensemble sampler sets on its own handles
     if case["op"] == "eval":
         sd.add_obs_array(inp["X"])
         if case["fit"]:
