@@ -128,7 +128,7 @@ struct nckde
   std::mutex mtx;
 
   // prepared device state
-  DBuf dX, dY, dcovg, dUg, dlng, dcov, dU, dinfo, dlnnorm, dw, db, dWp, dTh, dknn, dkeys, dscratch, dstatus,
+  DBuf dX, dY, dcovg, dUg, dlng, dcov, dU, dinfo, dlnnorm, dw, db, dterm, dWp, dTh, dknn, dkeys, dscratch, dstatus,
        dwcum, dwhich;
   // mixed-precision factors (built at the first mixed eval after a prepare)
   DBuf dmu, dYc, dymax, dA16, dc32, dcoef, dYw, dpartMf, dflag;
@@ -473,6 +473,8 @@ refresh_bvec (nckde *h)
   HIPCHK (h->db.ensure (sizeof (double) * h->n_k));
   HIPCHK (nck::launch_bvec (h->dw.as<double> (), (h->kind == NCKDE_VKDE) ? h->dlnnorm.as<double> () : nullptr,
                             (int) h->n_k, h->db.as<double> (), h->stream));
+  HIPCHK (h->dterm.ensure (sizeof (double) * (h->n_k + 1)));
+  HIPCHK (nck::launch_eval_terms (h->db.as<double> (), (int) h->n_k, h->kernel, h->dterm.as<double> (), h->stream));
   h->wcum_ready    = false;
   h->mixed_b_ready = false;
   h->f32_b_ready   = false;
@@ -607,6 +609,7 @@ build_IM (nckde *h, const double *dm2lnp, double min_m2lnp)
   a.m2lnp       = dm2lnp;
   a.min_m2lnp   = min_m2lnp;
   a.AT          = h->dAT.as<double> ();
+  a.pw          = nck::half_power_of (h->kernel, h->nu, h->d);
 
   HIPCHK (nck::launch_build_IM (a, h->stream));
 
@@ -1792,6 +1795,10 @@ eval_fp64_ws (nckde *h, const double *dX, size_t m, double *dout, int linear, hi
   a.nsplit        = nsplit;
   a.out           = dout;
   a.linear        = linear;
+  a.term          = h->dterm.as<double> ();
+  a.tref          = h->dterm.as<double> () + h->n_k;
+  a.pw            = nck::half_power_of (h->kernel, h->nu, h->d);
+  a.fc            = (h->kernel == NCKDE_KERNEL_GAUSS) ? -0.5 * nck::LOG2E_D * a.inv_h2 : a.inv_h2 / h->nu;
 
   if (f32)
   {

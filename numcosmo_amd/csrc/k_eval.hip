@@ -14,16 +14,29 @@
 // (eval_weights_m2lnp), the sum0/sum1 reductions of
 // ncm_stats_dist_kernel_gauss.c:246-333 / ncm_stats_dist_kernel_st.c:295-386
 // and the linear eval_weights (vkde.c:631-679, kde.c:596-637).
+#include "kde_math.h"
 #include "nckde_internal.h"
 
 namespace nck
 {
 
+// Smallest sum of a split that the fast form below may return: above it the
+// terms lost to underflow (under 1e-308) cannot be seen.
+constexpr double FAST_FLOOR = 1.0e-250;
+
+// The terms are formed in two ways.  Fast (Gauss, and Student-t with an
+// integer nu up to 127 - d): term_i K against the reference max_i b_i, which
+// every lane shares, K = 2^t or the (nu + d)-th power of an inverse square
+// root.  A lane whose sum is not a normal number in range (a point so far out
+// that its terms underflow, NaN or inf input) runs the general form instead:
+// ln K with log1p, and an online maximum.  The logarithm, the exponential and
+// the maximum of the general form cost as much as the 136 FMAs of a d = 16
+// factor.
 template <int D, int KERNEL, int KIND>
 __global__ void __launch_bounds__ (256)
 k_eval_f64 (EvalArgs a)
 {
-  const int p     = blockIdx.x * 256 + threadIdx.x;
+  const int p     = blockIdx.x * blockDim.x + threadIdx.x;
   const int chunk = (a.n + a.nsplit - 1) / a.nsplit;
   const int i0    = blockIdx.y * chunk;
   const int i1    = min (a.n, i0 + chunk);
@@ -80,10 +93,8 @@ k_eval_f64 (EvalArgs a)
       x[l] = v[l];
   }
 
-  double M = -INFINITY, S = 0.0;
-
-  for (int i = i0; i < i1; ++i)
-  {
+  // |W_i (x - theta_i)|^2, before the bandwidth
+  auto chi2_of = [&] (int i) -> double {
     const double *th = a.Th + (size_t) i * D;
     double chi2      = 0.0;
 
@@ -99,6 +110,9 @@ k_eval_f64 (EvalArgs a)
 #pragma unroll
       for (int r = 0; r < D; ++r)
       {
+        if (row_guard (D, r) && r >= d)
+          break;
+
         double z = 0.0;
 
 #pragma unroll
@@ -119,25 +133,56 @@ k_eval_f64 (EvalArgs a)
       }
     }
 
-    chi2 *= a.inv_h2;
+    return chi2;
+  };
 
-    double lnt;
+  double M  = -INFINITY, S = 0.0;
+  bool done = false;
 
-    if (KERNEL == NCKDE_KERNEL_GAUSS)
-      lnt = fma (-0.5, chi2, a.b[i]);
-    else
-      lnt = fma (a.kappa, log1p (chi2 / a.nu), a.b[i]);
-
-    if (lnt > M)
+  // the terms against the common reference max_i b_i, without logarithm or
+  // running maximum
+  if (KERNEL == NCKDE_KERNEL_GAUSS || a.pw > 0)
+  {
+    for (int i = i0; i < i1; ++i)
     {
-      S = S * exp (M - lnt);
-      M = lnt;
+      const double chi2 = chi2_of (i);
+
+      if (KERNEL == NCKDE_KERNEL_GAUSS)
+        S += exp2_f64 (fma (chi2, a.fc, a.term[i]));
+      else
+        S = fma (a.term[i], half_power (fma (chi2, a.fc, 1.0), a.pw), S);
     }
 
-    {
-      const double e = exp (lnt - M);
+    done = (S > FAST_FLOOR) && (S < INFINITY);
+    M    = *a.tref;
+  }
 
-      S += (lnt > -INFINITY) ? e : 0.0;
+  if (!done)
+  {
+    M = -INFINITY;
+    S = 0.0;
+
+    for (int i = i0; i < i1; ++i)
+    {
+      const double chi2 = chi2_of (i) * a.inv_h2;
+      double lnt;
+
+      if (KERNEL == NCKDE_KERNEL_GAUSS)
+        lnt = fma (-0.5, chi2, a.b[i]);
+      else
+        lnt = fma (a.kappa, log1p (chi2 / a.nu), a.b[i]);
+
+      if (lnt > M)
+      {
+        S = S * exp (M - lnt);
+        M = lnt;
+      }
+
+      {
+        const double e = exp (lnt - M);
+
+        S += (lnt > -INFINITY) ? e : 0.0;
+      }
     }
   }
 
@@ -158,7 +203,7 @@ template <int D, int KERNEL, int KIND>
 __global__ void __launch_bounds__ (256)
 k_eval_f32 (EvalArgs a)
 {
-  const int p     = blockIdx.x * 256 + threadIdx.x;
+  const int p     = blockIdx.x * blockDim.x + threadIdx.x;
   const int chunk = (a.n + a.nsplit - 1) / a.nsplit;
   const int i0    = blockIdx.y * chunk;
   const int i1    = min (a.n, i0 + chunk);
@@ -307,46 +352,130 @@ launch_f32_b2 (const double *b, double bref, int n, float *b2f, hipStream_t s)
   return hipGetLastError ();
 }
 
-// gamma = max over splits, 1 + lambda = sum_s S_s exp(M_s - gamma);
-// m2lnp = -2 (gamma - lnnorm_shared + log1p(lambda) - d ln h)
-__global__ void
-k_eval_merge (EvalArgs a)
+// gamma = max over splits, S = sum_s S_s exp(M_s - gamma);
+// m2lnp = -2 (gamma - lnnorm_shared + ln S - d ln h)
+//
+// A block takes 256 / L points with L lanes each.  Lane l takes the splits l,
+// l + L, ...; the lanes' maxima and sums combine as a tree in LDS, so the
+// result depends on nsplit and L only.  The reads of the partials bound it:
+// 8 lanes keep 256-byte rows coalesced over 32 points and are used from 2048
+// points on; below, 64 lanes (256 up to 64 points) shorten the serial walk
+// over the splits, which one lane per point ran in 66 us at m = 6400.
+__global__ void __launch_bounds__ (256)
+k_eval_merge (EvalArgs a, int L)
 {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ double red[256];
+  const int np = 256 / L;
+  const int pl = threadIdx.x % np, sl = threadIdx.x / np;
+  const int p  = blockIdx.x * np + pl;
+  const int pp = (p < a.m) ? p : a.m - 1;
+  double M     = -INFINITY;
 
-  if (p >= a.m)
-    return;
+  for (int s = sl; s < a.nsplit; s += L)
+    M = fmax (M, a.partM[(size_t) s * a.m + pp]);
 
-  double M = -INFINITY;
+  red[threadIdx.x] = M;
+  __syncthreads ();
 
-  for (int s = 0; s < a.nsplit; ++s)
-    M = fmax (M, a.partM[(size_t) s * a.m + p]);
+  for (int o = L / 2; o > 0; o >>= 1)
+  {
+    if (sl < o)
+      red[threadIdx.x] = fmax (red[threadIdx.x], red[threadIdx.x + o * np]);
+
+    __syncthreads ();
+  }
+
+  M = red[pl];
+  __syncthreads ();
 
   double S = 0.0;
 
-  for (int s = 0; s < a.nsplit; ++s)
+  for (int s = sl; s < a.nsplit; s += L)
   {
-    const double Ms = a.partM[(size_t) s * a.m + p];
+    const double Ms = a.partM[(size_t) s * a.m + pp];
+    const double Ss = a.partS[(size_t) s * a.m + pp];
 
-    if (Ms > -INFINITY)
-      S += a.partS[(size_t) s * a.m + p] * exp (Ms - M);
+    if (Ms == M)
+      S += (M > -INFINITY) ? Ss : 0.0;
+    else if (Ms > -INFINITY)
+      S += Ss * exp (Ms - M);
   }
 
-  const double m2lnp = -2.0 * ((M - a.lnnorm_shared) + log1p (S - 1.0) - a.lnh_d);
+  red[threadIdx.x] = S;
+  __syncthreads ();
+
+  for (int o = L / 2; o > 0; o >>= 1)
+  {
+    if (sl < o)
+      red[threadIdx.x] += red[threadIdx.x + o * np];
+
+    __syncthreads ();
+  }
+
+  if (sl != 0 || p >= a.m)
+    return;
+
+  const double m2lnp = -2.0 * ((M - a.lnnorm_shared) + log (red[pl]) - a.lnh_d);
 
   a.out[p] = a.linear ? exp (-0.5 * m2lnp) : m2lnp;
+}
+
+// The per-kernel constants of the fast form against bref = max_i b_i:
+// Student-t term_i = exp (b_i - bref), Gauss term_i = (b_i - bref) log2 e;
+// term[n] = bref.  One block: the arrays are n doubles.
+__global__ void __launch_bounds__ (1024)
+k_eval_terms (const double *__restrict__ b, int n, int kernel, double *__restrict__ term)
+{
+  __shared__ double red[1024];
+  double M = -INFINITY;
+
+  for (int i = threadIdx.x; i < n; i += 1024)
+    M = fmax (M, b[i]);
+
+  red[threadIdx.x] = M;
+  __syncthreads ();
+
+  for (int o = 512; o > 0; o >>= 1)
+  {
+    if (threadIdx.x < o)
+      red[threadIdx.x] = fmax (red[threadIdx.x], red[threadIdx.x + o]);
+
+    __syncthreads ();
+  }
+
+  M = red[0];
+
+  for (int i = threadIdx.x; i < n; i += 1024)
+  {
+    const double t = b[i] - M;
+
+    term[i] = (kernel == NCKDE_KERNEL_GAUSS) ? t * 1.4426950408889634073599246810018921 : exp (t);
+  }
+
+  if (threadIdx.x == 0)
+    term[n] = M;
+}
+
+hipError_t
+launch_eval_terms (const double *b, int n, int kernel, double *term, hipStream_t s)
+{
+  hipLaunchKernelGGL (k_eval_terms, dim3 (1), dim3 (1024), 0, s, b, n, kernel, term);
+
+  return hipGetLastError ();
 }
 
 template <int D, int KERNEL, int KIND>
 static hipError_t
 launch_t (const EvalArgs &a, hipStream_t s)
 {
-  dim3 grid ((a.m + 255) / 256, a.nsplit);
+  // one wave holds up to 64 points: further waves of a block would repeat it
+  const int bs = (a.m <= 64) ? 64 : (a.m <= 128) ? 128 : 256;
+  dim3 grid ((a.m + bs - 1) / bs, a.nsplit);
 
   if (a.b2f != nullptr)
-    hipLaunchKernelGGL ((k_eval_f32<D, KERNEL, KIND>), grid, dim3 (256), 0, s, a);
+    hipLaunchKernelGGL ((k_eval_f32<D, KERNEL, KIND>), grid, dim3 (bs), 0, s, a);
   else
-    hipLaunchKernelGGL ((k_eval_f64<D, KERNEL, KIND>), grid, dim3 (256), 0, s, a);
+    hipLaunchKernelGGL ((k_eval_f64<D, KERNEL, KIND>), grid, dim3 (bs), 0, s, a);
 
   return hipGetLastError ();
 }
@@ -395,7 +524,9 @@ launch_eval_f64 (const EvalArgs &a, hipStream_t s)
 hipError_t
 launch_eval_merge (const EvalArgs &a, hipStream_t s)
 {
-  hipLaunchKernelGGL (k_eval_merge, dim3 ((a.m + 255) / 256), dim3 (256), 0, s, a);
+  const int L = (a.m >= 2048) ? 8 : (a.m > 64) ? 64 : 256;
+
+  hipLaunchKernelGGL (k_eval_merge, dim3 ((a.m + 256 / L - 1) / (256 / L)), dim3 (256), 0, s, a, L);
 
   return hipGetLastError ();
 }

@@ -8,6 +8,7 @@
 // Reference: _ncm_stats_dist_compute_IM_full (ncm_stats_dist.c:791-804),
 // compute_IM (ncm_stats_dist_kde.c:492-557, ncm_stats_dist_vkde.c:517-606),
 // ncm_nnls_solve and its normal-equation solvers (ncm_nnls.c:464-871).
+#include "kde_math.h"
 #include "nckde_internal.h"
 
 namespace nck
@@ -96,6 +97,9 @@ k_build_IM (IMArgs a, const double *__restrict__ Wp, const double *__restrict__ 
 #pragma unroll
         for (int r = 0; r < D; ++r)
         {
+          if (row_guard (D, r) && r >= d)
+            break;
+
           double z = 0.0;
 
 #pragma unroll
@@ -124,8 +128,12 @@ k_build_IM (IMArgs a, const double *__restrict__ Wp, const double *__restrict__ 
 
       double K;
 
+      const double u = fma (chi2, inv_nu, 1.0);
+
       if (KERNEL == NCKDE_KERNEL_GAUSS)
         K = exp (-0.5 * chi2);
+      else if (a.pw > 0 && u < 1.0e290)
+        K = half_power (u, a.pw);
       else
         K = exp (kappa * log1p (chi2 * inv_nu));
 

@@ -29,6 +29,7 @@
 namespace nck
 {
 
+constexpr double LOG2E_D = 1.4426950408889634073599246810018921;
 constexpr double LN2PI = 1.8378770664093454835606594728112353;
 constexpr double LNPI  = 1.1447298858494001741434273513530587;
 constexpr double LOG_DBL_EPSILON = -3.6043653389117154e+01;
@@ -178,6 +179,12 @@ struct EvalArgs
   int nsplit;
   double *out;                     // m
   int linear;                      // 0: m2lnp, 1: density
+  // fast form of the FP64 terms (k_eval_terms): per-kernel constants against
+  // *tref = max_i b_i; fc = -log2(e) / (2 h^2) (Gauss) or 1 / (nu h^2)
+  // (Student-t); pw = nu + d for an integer nu, else 0 (general form only)
+  const double *term = nullptr, *tref = nullptr;
+  double fc          = 0.0;
+  int pw             = 0;
   // FP32 rung (b2f != NULL): FP32 factors (VKDE), b_i - bref in FP32
   const float *Wf = nullptr, *b2f = nullptr;
   double bref     = 0.0;
@@ -187,6 +194,15 @@ hipError_t launch_eval_f64 (const EvalArgs &a, hipStream_t s);
 hipError_t launch_f32_factors (const double *Wp, size_t count, float *Wf, hipStream_t s);
 hipError_t launch_f32_b2 (const double *b, double bref, int n, float *b2f, hipStream_t s);
 hipError_t launch_eval_merge (const EvalArgs &a, hipStream_t s);
+// term: n + 1 doubles (the last one max_i b_i)
+hipError_t launch_eval_terms (const double *b, int n, int kernel, double *term, hipStream_t s);
+// nu + d when the Student-t kernel is an integer power of rsqrt (1 + chi2 /
+// nu) that half_power takes, else 0
+inline int
+half_power_of (int kernel, double nu, int d)
+{
+  return (kernel == NCKDE_KERNEL_ST && nu >= 1.0 && nu + d <= 127.0 && nu == (double) (int) nu) ? (int) nu + d : 0;
+}
 
 // ---- mixed-precision evaluation (k_eval_mixed.hip) ------------------------
 struct MixedFactors
@@ -262,6 +278,7 @@ struct IMArgs
   const double *m2lnp;     // NULL: no row scaling
   double min_m2lnp;
   double *AT;              // n_k x n_obs (column-major A)
+  int pw = 0;              // half_power_of the kernel
 };
 hipError_t launch_build_IM (const IMArgs &a, hipStream_t s);
 hipError_t launch_transpose (const double *in, int rows, int cols, double *out, hipStream_t s);

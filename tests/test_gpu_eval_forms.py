@@ -1,0 +1,86 @@
+"""The two forms of the FP64 per-pair terms (a power of an inverse square root
+or 2^t against a common reference; ln K with an online maximum) and the merge
+of the split sums, against the FP64 oracle at the sizes where they change:
+integer and non-integer nu, the largest power taken, dimensions around the
+padded ones, points whose terms underflow, and point counts around the block
+and merge layouts.  Bar: 1e-12 relative (the terms' rounding, |ln K| ulps of
+each, averages below 1e-14; the bar of the other FP64 eval tests).
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _pair(oracle, kind, nu, d, X):
+    import numcosmo_amd as na
+    sdk = na.StatsDistKernelGauss.new(d) if nu == 0.0 else na.StatsDistKernelST.new(d, nu)
+    sd = (na.StatsDistVKDE if kind == 1 else na.StatsDistKDE).new(sdk, na.StatsDistCV.NONE)
+    od = oracle.StatsDist(kind, 0 if nu == 0.0 else 1, d, nu)
+    for o in (sd, od):
+        if kind == 1:
+            o.set_local_frac(0.4)
+        o.add_obs_array(X)
+        o.prepare()
+    return sd, od
+
+
+def _check(sd, od, P):
+    got, ref = sd.eval_m2lnp_batch(P, 0), od.eval_m2lnp_batch(P)
+    assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-12
+
+
+@pytest.mark.parametrize("kind", [0, 1])
+@pytest.mark.parametrize("nu", [0.0, 1.0, 2.0, 2.5, 3.0])
+@pytest.mark.parametrize("d", [1, 3, 4, 5, 6, 7, 12, 13, 15, 16, 17, 20, 21, 24, 25, 29, 33, 37, 48, 49, 53, 57, 64])
+def test_forms_by_dimension(oracle, kind, nu, d):
+    g = np.random.default_rng(d)
+    n = 3 * d + 40
+    X = g.normal(size=(n, d))
+    sd, od = _pair(oracle, kind, nu, d, X)
+    P = np.concatenate([X[:5], g.normal(size=(60, d)), 30.0 * g.normal(size=(5, d))])
+    _check(sd, od, P)
+
+
+@pytest.mark.parametrize("nu", [122.0, 123.0, 124.0, 0.0, 5.0])
+def test_largest_power_and_underflow(oracle, nu):
+    """nu + d = 126, 127 (fast), 128 (general); far points whose terms all
+    underflow against the common reference."""
+    g = np.random.default_rng(3)
+    X = g.normal(size=(200, 4))
+    sd, od = _pair(oracle, 1, nu, 4, X)
+    P = np.concatenate([g.normal(size=(50, 4)) * s for s in (1.0, 1e2, 1e5, 1e9)])
+    _check(sd, od, P)
+
+
+@pytest.mark.parametrize("nu", [0.0, 2.5, 3.0])
+@pytest.mark.parametrize("d", [5, 16, 33])
+def test_non_finite_points(oracle, nu, d):
+    """A point with NaN or inf has density 0 (m2lnp = +inf) and leaves the
+    points beside it alone."""
+    g = np.random.default_rng(4)
+    X = g.normal(size=(160, d))
+    sd, od = _pair(oracle, 1, nu, d, X)
+    P = g.normal(size=(70, d))
+    clean = sd.eval_m2lnp_batch(P, 0)
+    Q = P.copy()
+    Q[3, 0] = np.nan
+    Q[17, d - 1] = np.inf
+    Q[69, d // 2] = -np.inf
+    got = sd.eval_m2lnp_batch(Q, 0)
+    bad = [3, 17, 69]
+    assert np.all(np.isposinf(got[bad]))
+    keep = np.setdiff1d(np.arange(70), bad)
+    assert np.array_equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("m", [1, 2, 63, 64, 65, 128, 129, 255, 257, 2047, 2048, 2049])
+@pytest.mark.parametrize("d", [3, 16, 40])
+@pytest.mark.parametrize("precision", [0, 2])
+def test_point_counts(oracle, m, d, precision):
+    g = np.random.default_rng(m)
+    X = g.normal(size=(333, d))
+    sd, od = _pair(oracle, 1, 3.0, d, X)
+    P = g.normal(size=(m, d))
+    got, ref = sd.eval_m2lnp_batch(P, precision), od.eval_m2lnp_batch(P)
+    assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < (1e-12 if precision == 0 else 1e-6)
