@@ -20,10 +20,6 @@
 namespace nck
 {
 
-// Smallest sum of a split that the fast form below may return: above it the
-// terms lost to underflow (under 1e-308) cannot be seen.
-constexpr double FAST_FLOOR = 1.0e-250;
-
 // The terms are formed in two ways.  Fast (Gauss, and Student-t with an
 // integer nu up to 127 - d): term_i K against the reference max_i b_i, which
 // every lane shares, K = 2^t or the (nu + d)-th power of an inverse square
@@ -42,27 +38,12 @@ k_eval_f64 (EvalArgs a)
   const int i1    = min (a.n, i0 + chunk);
   const int pp    = (p < a.m) ? p : (a.m - 1);
   const int d     = a.d;
-  // VKDE at D = 64: the point is read again for every kernel (from L1/L2)
-  // instead of being held beside the differences, which left one wave per
-  // SIMD (1.5x as long at n = 8000, m = 20000; at D = 32, and in the FP32
-  // rung, the re-reads cost more than the occupancy gains).  KDE keeps its
-  // whitened point in registers.
-  constexpr bool XREG = (KIND == NCKDE_KDE) || (D < 64);
-  const double *xrow  = a.X + (size_t) pp * d;
-  double x[XREG ? D : 1];
-  auto xv = [&] (int k) -> double {
-    if constexpr (XREG)
-      return x[k];
-    else
-      return (k < d) ? xrow[k] : 0.0;
-  };
+  const double *xrow = a.X + (size_t) pp * d;
+  double x[D];
 
-  if constexpr (XREG)
-  {
 #pragma unroll
-    for (int k = 0; k < D; ++k)
-      x[k] = (k < d) ? xrow[k] : 0.0;
-  }
+  for (int k = 0; k < D; ++k)
+    x[k] = (k < d) ? xrow[k] : 0.0;
 
   if constexpr (KIND == NCKDE_KDE)
   {
@@ -105,7 +86,7 @@ k_eval_f64 (EvalArgs a)
 
 #pragma unroll
       for (int k = 0; k < D; ++k)
-        delta[k] = xv (k) - th[k];
+        delta[k] = x[k] - th[k];
 
 #pragma unroll
       for (int r = 0; r < D; ++r)
@@ -127,7 +108,7 @@ k_eval_f64 (EvalArgs a)
 #pragma unroll
       for (int k = 0; k < D; ++k)
       {
-        const double t = th[k] - xv (k);
+        const double t = th[k] - x[k];
 
         chi2 = fma (t, t, chi2);
       }
@@ -153,7 +134,7 @@ k_eval_f64 (EvalArgs a)
         S = fma (a.term[i], half_power (fma (chi2, a.fc, 1.0), a.pw), S);
     }
 
-    done = (S > FAST_FLOOR) && (S < INFINITY);
+    done = (S > EVAL_FAST_FLOOR) && (S < INFINITY);
     M    = *a.tref;
   }
 
@@ -273,11 +254,6 @@ k_eval_f32 (EvalArgs a)
           z = fmaf (W[r * (r + 1) / 2 + c], delta[c], z);
 
         chi2 = fmaf (z, z, chi2);
-
-        // one row's factor entries live at a time: without the fence the
-        // scalar loads of every row are hoisted together and spill at D >= 32
-        if (D >= 32)
-          __builtin_amdgcn_sched_barrier (0);
       }
     }
     else
@@ -484,9 +460,10 @@ template <int D>
 static hipError_t
 launch_d (const EvalArgs &a, hipStream_t s)
 {
-  if (a.kind == NCKDE_VKDE)
-    return (a.kernel == NCKDE_KERNEL_GAUSS) ? launch_t<D, NCKDE_KERNEL_GAUSS, NCKDE_VKDE> (a, s)
-                                            : launch_t<D, NCKDE_KERNEL_ST, NCKDE_VKDE> (a, s);
+  if constexpr (D < TILE_MIN_D)
+    if (a.kind == NCKDE_VKDE)
+      return (a.kernel == NCKDE_KERNEL_GAUSS) ? launch_t<D, NCKDE_KERNEL_GAUSS, NCKDE_VKDE> (a, s)
+                                              : launch_t<D, NCKDE_KERNEL_ST, NCKDE_VKDE> (a, s);
 
   return (a.kernel == NCKDE_KERNEL_GAUSS) ? launch_t<D, NCKDE_KERNEL_GAUSS, NCKDE_KDE> (a, s)
                                           : launch_t<D, NCKDE_KERNEL_ST, NCKDE_KDE> (a, s);
@@ -507,6 +484,9 @@ padded_dim (int d)
 hipError_t
 launch_eval_f64 (const EvalArgs &a, hipStream_t s)
 {
+  if (a.kind == NCKDE_VKDE && a.d >= TILE_MIN_D)
+    return launch_eval_tile (a, s);
+
   switch (a.D)
   {
     case 4: return launch_d<4> (a, s);

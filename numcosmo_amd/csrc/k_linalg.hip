@@ -40,9 +40,8 @@ k_build_IM (IMArgs a, const double *__restrict__ Wp, const double *__restrict__ 
   const bool live = (j < a.n_obs);
   const int jj    = live ? j : (a.n_obs - 1);
   const int d     = a.d;
-  // at D >= 32 the point is read again for every kernel (from L1/L2): held
-  // in registers beside the differences it left one wave per SIMD at D = 64
-  // and two at D = 32 (the build took 2.0x and 1.5x as long)
+  // at D >= 32 the point is read again for every kernel (from L1/L2) instead
+  // of being held in registers beside the differences
   constexpr bool XREG = (D < 32);
   const double *xrow  = ((KIND == NCKDE_VKDE) ? a.X : a.Y) + (size_t) jj * d;
   double xj[XREG ? D : 1];
@@ -181,9 +180,10 @@ template <int D>
 static hipError_t
 im_d (const IMArgs &a, hipStream_t s)
 {
-  if (a.kind == NCKDE_VKDE)
-    return (a.kernel == NCKDE_KERNEL_GAUSS) ? im_t<D, NCKDE_KERNEL_GAUSS, NCKDE_VKDE> (a, s)
-                                            : im_t<D, NCKDE_KERNEL_ST, NCKDE_VKDE> (a, s);
+  if constexpr (D < TILE_MIN_D)
+    if (a.kind == NCKDE_VKDE)
+      return (a.kernel == NCKDE_KERNEL_GAUSS) ? im_t<D, NCKDE_KERNEL_GAUSS, NCKDE_VKDE> (a, s)
+                                              : im_t<D, NCKDE_KERNEL_ST, NCKDE_VKDE> (a, s);
 
   return (a.kernel == NCKDE_KERNEL_GAUSS) ? im_t<D, NCKDE_KERNEL_GAUSS, NCKDE_KDE> (a, s)
                                           : im_t<D, NCKDE_KERNEL_ST, NCKDE_KDE> (a, s);
@@ -192,6 +192,9 @@ im_d (const IMArgs &a, hipStream_t s)
 hipError_t
 launch_build_IM (const IMArgs &a, hipStream_t s)
 {
+  if (a.kind == NCKDE_VKDE && a.d >= TILE_MIN_D)
+    return launch_im_tile (a, s);
+
   switch (a.D)
   {
     case 4: return im_d<4> (a, s);

@@ -189,6 +189,13 @@ struct EvalArgs
   const float *Wf = nullptr, *b2f = nullptr;
   double bref     = 0.0;
 };
+// Smallest sum of a split that the fast form of the FP64 terms may return:
+// above it the terms lost to underflow (under 1e-308) cannot be seen.
+constexpr double EVAL_FAST_FLOOR = 1.0e-250;
+// dimension from which the VKDE's per-pair products run on the matrix cores
+// (k_eval_tile.hip, k_im_tile.hip)
+constexpr int TILE_MIN_D = 13;
+hipError_t launch_eval_tile (const EvalArgs &a, hipStream_t s);
 // FP64 eval, or the FP32 rung when a.b2f is set
 hipError_t launch_eval_f64 (const EvalArgs &a, hipStream_t s);
 hipError_t launch_f32_factors (const double *Wp, size_t count, float *Wf, hipStream_t s);
@@ -281,6 +288,7 @@ struct IMArgs
   int pw = 0;              // half_power_of the kernel
 };
 hipError_t launch_build_IM (const IMArgs &a, hipStream_t s);
+hipError_t launch_im_tile (const IMArgs &a, hipStream_t s);
 hipError_t launch_transpose (const double *in, int rows, int cols, double *out, hipStream_t s);
 hipError_t launch_gram_nt (const double *AT, int n, int K, double *M, hipStream_t s);
 hipError_t launch_row_dot (const double *AT, int n, int K, const double *v, double *out, hipStream_t s);

@@ -84,3 +84,16 @@ def test_point_counts(oracle, m, d, precision):
     P = g.normal(size=(m, d))
     got, ref = sd.eval_m2lnp_batch(P, precision), od.eval_m2lnp_batch(P)
     assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < (1e-12 if precision == 0 else 1e-6)
+
+
+@pytest.mark.parametrize("nu", [0.0, 2.5, 3.0])
+@pytest.mark.parametrize("d,n", [(5, 70), (12, 257), (13, 64), (16, 129), (17, 300), (24, 320), (36, 333), (64, 515)])
+def test_interpolation_matrix(oracle, nu, d, n):
+    """IM of the vector and the matrix-core forms: kernels and observations
+    that leave partial tiles.  1e-11: chi2 reaches 1e3 on the outer pairs and
+    ln K turns its 1e-15 relative error into 1e-12 of K."""
+    g = np.random.default_rng(d + n)
+    X = g.normal(size=(n, d))
+    sd, od = _pair(oracle, 1, nu, d, X)
+    got, ref = sd.compute_IM(), od.compute_IM()
+    assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1e-300)) < 1e-11
