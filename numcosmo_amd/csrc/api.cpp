@@ -728,22 +728,22 @@ nnls_hstat (nckde *h)
 // slot of the pinned statistics that receives the chained sweeps' status
 constexpr int TRSV_STATUS_SLOT = 6;
 
-// (U^T U) x = b with the factor in dS and b in dbs: the flag-chained sweeps
+// U x = y with the factor in dS, y in dtv and x in dbs: the flag-chained sweep
 // when every panel block fits on the device at once, else one launch per
-// panel.  A chained solve's status is read with the caller's next read-back
+// panel.  A chained sweep's status is read with the caller's next read-back
 // (trsv_pending holds its epoch).
 static int
-nnls_trsv (nckde *h, int np, hipStream_t s)
+nnls_backward (nckde *h, int np, hipStream_t s)
 {
   const int npan = (np + 63) / 64;
 
   if (h->trsv_chain_off || npan > nck::trsv_chain_max_panels ())
   {
-    HIPCHK (nck::launch_trsv_pair (h->dS.as<double> (), np, h->dbs.as<double> (), h->dtv.as<double> (), s));
+    HIPCHK (nck::launch_trsv_backward (h->dS.as<double> (), np, h->dtv.as<double> (), h->dbs.as<double> (), s));
     return NCKDE_OK;
   }
 
-  const size_t words = 1 + 2 * (size_t) npan;
+  const size_t words = 1 + (size_t) npan;
 
   if (words > h->flags_words || h->trsv_epoch == 0xffffffffu)
   {
@@ -755,7 +755,7 @@ nnls_trsv (nckde *h, int np, hipStream_t s)
 
   const unsigned epoch = ++h->trsv_epoch;
 
-  HIPCHK (nck::launch_trsv_chain (h->dS.as<double> (), np, h->dbs.as<double> (), h->dtv.as<double> (),
+  HIPCHK (nck::launch_trsv_chain (h->dS.as<double> (), np, h->dtv.as<double> (), h->dbs.as<double> (),
                                   h->dtsflags.as<unsigned> (), epoch, s));
   HIPCHK (hipMemcpyAsync (nnls_hstat (h) + TRSV_STATUS_SLOT, h->dtsflags.p, sizeof (unsigned), hipMemcpyDeviceToHost,
                           s));
@@ -819,10 +819,11 @@ nnls_unconstrained (nckde *h, int n, const std::vector<int> &P, double *dxo)
     } st = {0, 0, 0.0, 0.0};
 
     HIPCHK (nck::launch_gather_sym (h->dM.as<double> (), n, h->dP.as<int> (), np, h->dS.as<double> (),
-                                    h->dbv.as<double> (), h->dbs.as<double> (), s));
+                                    h->dbv.as<double> (), h->dtv.as<double> (), s));
     HIPCHK (hipMemsetAsync (h->dscal.p, 0, sizeof (int) * 2, s));
     HIPCHK (h->dpd.ensure (sizeof (double) * nck::potrf_diag_doubles (np)));
-    HIPCHK (nck::launch_potrf (h->dS.as<double> (), np, h->dscal.as<int> (), h->dpd.as<double> (), s));
+    HIPCHK (nck::launch_potrf (h->dS.as<double> (), np, h->dtv.as<double> (), h->dscal.as<int> (),
+                               h->dpd.as<double> (), s));
     HIPCHK (nck::launch_diag_range (h->dS.as<double> (), np, h->dscal.as<double> () + 1, s));
     HIPCHK (hipMemcpyAsync (nnls_hstat (h), h->dscal.p, sizeof (st), hipMemcpyDeviceToHost, s));
     HIPCHK (hipStreamSynchronize (s));
@@ -830,7 +831,7 @@ nnls_unconstrained (nckde *h, int n, const std::vector<int> &P, double *dxo)
 
     if (st.info == 0)
     {
-      TRY (nnls_trsv (h, np, s));
+      TRY (nnls_backward (h, np, s));
       h->nnls_rungs[0]++;
 
       if (h->nnls_refine > 0 && st.dmax * st.dmax >= REFINE_PIVOT_RATIO * st.dmin * st.dmin)

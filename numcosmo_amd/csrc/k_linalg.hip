@@ -258,9 +258,9 @@ launch_transpose (const double *in, int rows, int cols, double *out, hipStream_t
 //   mode 0: M = AT AT^T (AT is n x K row-major): the Gram matrix A^T A of
 //           the NNLS normal equations (cblas_dsyrk, ncm_matrix.c:1547-1575);
 //           both triangles are written.
-//   mode 1: trailing update of the blocked Cholesky, S[a][b] -= sum_r
-//           S[kb+r][a] S[kb+r][b] over the panel rows kb..kb+K-1, for
-//           off <= a <= b (upper triangle only).
+//   mode 1: trailing update of the Cholesky's super-panels (k_potrf.hip),
+//           S[a][b] -= sum_r S[kb+r][a] S[kb+r][b] over the rows
+//           kb..kb+K-1, for off <= a <= b (upper triangle only).
 // Tiles are numbered along the rows of the upper triangle; the grid is
 // padded to a multiple of 8 and block b takes tile (b % 8) * (grid / 8) +
 // b / 8, so that each XCD (blocks are dealt round-robin over the 8 XCDs)
@@ -461,15 +461,12 @@ k_syrk_mfma (const double *__restrict__ P, int n, int K, int ld, int off, int kb
   }
 }
 
-// row_end > 0: only the tile rows below row_end (row_end - off a multiple
-// of BM), every column from the tile row on
 template <int MODE, int BM = SY_BM>
 static void
-launch_syrk_mfma (const double *P, int n, int K, int ld, int off, int kb, double *M, hipStream_t s, int row_end = 0)
+launch_syrk_mfma (const double *P, int n, int K, int ld, int off, int kb, double *M, hipStream_t s)
 {
   const int nt     = (n - off + BM - 1) / BM;
-  const int nr     = (row_end > 0) ? (row_end - off + BM - 1) / BM : nt;
-  const int ntiles = nr * nt - nr * (nr - 1) / 2;
+  const int ntiles = nt * (nt + 1) / 2;
   const int grid   = (ntiles + 7) / 8 * 8;
 
   if (ntiles > 0)
@@ -705,207 +702,6 @@ launch_gather_sym (const double *M, int n, const int *P, int np, double *S, cons
   return hipGetLastError ();
 }
 
-// --------------------------------------------------------------------------
-// Blocked right-looking Cholesky of the SPD system S = U^T U (upper, as
-// dposv with the row-major 'U' of ncm_matrix.c:1198-1208), 64-wide panels:
-//   diagonal block in LDS (dot-product form), row-panel triangular solve,
-//   trailing rank-64 update of the upper triangle.
-// info = first failing global pivot + 1 (LAPACK convention), else 0.
-// --------------------------------------------------------------------------
-constexpr int CH_NB = 64;
-
-// Factor of the 64 x 64 diagonal block, right-looking with the block in
-// registers: thread (tr, tc) of a 16 x 16 grid owns entries
-// (tr + 16 a, tc + 16 b), a, b < 4.  Per column j the owner of (j, j)
-// publishes the pivot, the owners of row j publish the scaled row, and every
-// thread updates its own entries from two LDS vectors (two barriers per
-// column).  Returns the failing pivot + 1 (LAPACK info), else 0; every
-// thread of the block returns the same value.
-__device__ inline int
-factor_diag_block (const double *__restrict__ S, int np, int kb, int nb, double (&x)[4][4], double *row,
-                   double &piv)
-{
-  const int tid = threadIdx.x;
-  const int tr  = tid >> 4, tc = tid & 15;
-
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-    {
-      const int r = tr + 16 * a, c = tc + 16 * b;
-
-      x[a][b] = (r < nb && c < nb) ? S[(size_t) (kb + r) * np + kb + c] : 0.0;
-    }
-
-  for (int j = 0; j < nb; ++j)
-  {
-    const int ja = j >> 4, jr = j & 15;
-
-    if (tr == jr && tc == jr)
-    {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-        if (a == ja)
-          piv = x[a][a];
-    }
-
-    __syncthreads ();
-
-    const double djj = piv;
-
-    if (!(djj > 0.0))
-      return kb + j + 1;
-
-    const double ujj = sqrt (djj);
-
-    if (tr == jr)
-    {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-        if (a == ja)
-        {
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-          {
-            const int c = tc + 16 * b;
-
-            if (c >= j && c < nb)
-            {
-              const double u = (c == j) ? ujj : x[a][b] / ujj;
-
-              x[a][b] = u;
-              row[c]  = u;
-            }
-          }
-        }
-    }
-
-    __syncthreads ();
-
-    double ur[4], uc[4];
-
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-    {
-      const int r = tr + 16 * a, c = tc + 16 * a;
-
-      ur[a] = (r > j && r < nb) ? row[r] : 0.0;
-      uc[a] = (c > j && c < nb) ? row[c] : 0.0;
-    }
-
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        x[a][b] = fma (-ur[a], uc[b], x[a][b]);
-  }
-
-  return 0;
-}
-
-// Panel step for a panel narrower than 64 (the last one when np is not a
-// multiple of 64; full panels go through k_potrf_rowpanel): every block
-// factors the diagonal block (redundantly, from
-// the unfactored values, which stay in S until k_copy_diag), then solves
-// U_kk^T x = S[kb:kb+nb][c] for its 64 columns c >= kb+nb in LDS (wave 0, one
-// lane per column, four partial sums per row) and writes them back.  Block
-// 0 stores the factor in diagbuf.  Staging loads of the panel columns are
-// issued before the factorisation.
-__global__ void __launch_bounds__ (256)
-k_potrf_panel (double *__restrict__ S, int np, int kb, int nb, int *__restrict__ info, double *__restrict__ diagbuf)
-{
-  __shared__ double U[CH_NB][CH_NB + 1];
-  __shared__ double Xs[CH_NB][64 + 1];
-  __shared__ double row[CH_NB];
-  __shared__ double piv;
-  const int tid  = threadIdx.x;
-  const int tr   = tid >> 4, tc = tid & 15;
-  const int lane = tid & 63, w = tid >> 6;
-  const int c0   = kb + nb + blockIdx.x * 64;
-  const int c    = c0 + lane;
-
-  if (*info != 0)
-    return;
-
-  double vx[16];
-
-#pragma unroll
-  for (int q = 0; q < 16; ++q)
-  {
-    const int r = w * 16 + q;
-
-    vx[q] = (r < nb && c < np) ? S[(size_t) (kb + r) * np + c] : 0.0;
-  }
-
-  double x[4][4];
-  const int fail = factor_diag_block (S, np, kb, nb, x, row, piv);
-
-  if (fail)
-  {
-    if (blockIdx.x == 0 && tid == 0)
-      *info = fail;
-
-    return;
-  }
-
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-    {
-      const int r = tr + 16 * a, cc = tc + 16 * b;
-
-      if (r < nb && cc < nb)
-      {
-        U[r][cc] = x[a][b];
-
-        if (blockIdx.x == 0 && cc >= r)
-          diagbuf[r * CH_NB + cc] = x[a][b];
-      }
-    }
-
-#pragma unroll
-  for (int q = 0; q < 16; ++q)
-    Xs[w * 16 + q][lane] = vx[q];
-
-  __syncthreads ();
-
-  if (w == 0 && c0 < np)
-  {
-    for (int r = 0; r < nb; ++r)
-    {
-      double t0 = Xs[r][lane], t1 = 0.0, t2 = 0.0, t3 = 0.0;
-      int q     = 0;
-
-      for (; q + 4 <= r; q += 4)
-      {
-        t0 = fma (-U[q][r], Xs[q][lane], t0);
-        t1 = fma (-U[q + 1][r], Xs[q + 1][lane], t1);
-        t2 = fma (-U[q + 2][r], Xs[q + 2][lane], t2);
-        t3 = fma (-U[q + 3][r], Xs[q + 3][lane], t3);
-      }
-
-      for (; q < r; ++q)
-        t0 = fma (-U[q][r], Xs[q][lane], t0);
-
-      Xs[r][lane] = ((t0 + t1) + (t2 + t3)) / U[r][r];
-    }
-  }
-
-  __syncthreads ();
-
-  if (c < np)
-#pragma unroll
-    for (int q = 0; q < 16; ++q)
-    {
-      const int r = w * 16 + q;
-
-      if (r < nb)
-        S[(size_t) (kb + r) * np + c] = Xs[r][lane];
-    }
-}
-
 // double broadcast from lane `src` (a compile-time constant after unrolling)
 __device__ inline double
 bcast_lane (double v, int src)
@@ -914,145 +710,6 @@ bcast_lane (double v, int src)
   const int hi = __builtin_amdgcn_readlane (__double2hiint (v), src);
 
   return __hiloint2double (hi, lo);
-}
-
-// A full panel (nb = 64) is one launch: the diagonal block's factor and the
-// solve of the row panel right of it are one right-looking factorisation of
-// the 64 x (64 + cols) row panel, each column held whole by one lane (its
-// 64 entries in registers).  Block b has two waves: wave 0 holds the
-// diagonal block (every block factors it, from the same values with the
-// same arithmetic), wave 1 holds RP_EXTRA = 64 columns of the row panel.
-// Step j: wave 0 takes the pivot from lane j by readlane, forms u_jj =
-// sqrt(pivot) and r_j = 1 / u_jj, scales row j of the diagonal block by
-// r_j and publishes it with r_j in LDS (double-buffered, one barrier per
-// step); every lane of the row panel scales its own row-j entry by r_j; then
-// each lane applies the rank-one update a_i -= u_ji * u_jc to its rows i >
-// j, row j's entries read from LDS all at once.  Entries below the diagonal
-// take part in the diagonal block's updates unmasked: they only ever
-// combine with each other and are never stored.  A non-positive pivot is
-// recorded (the first one), the steps run on, and nothing is stored.  Two
-// waves per block measured fastest (2.0 ms for a 3200-column factor, against
-// 2.3 ms with four waves and 2.8 ms for a one-wave diagonal factor followed
-// by a separate panel solve): the step barrier is cheap between two waves.
-// The factor goes to Ud (upper triangle, row-major 64 x 64) and the
-// reciprocals of its diagonal to rd.
-constexpr int RP_EXTRA = 64;
-
-__global__ void __launch_bounds__ (64 + RP_EXTRA)
-k_potrf_rowpanel (double *__restrict__ S, int np, int kb, int *__restrict__ info, double *__restrict__ Ud,
-                  double *__restrict__ rd)
-{
-  __shared__ double R[2][CH_NB];
-  __shared__ double Rr[2];
-  __shared__ int s_fail;
-  const int tid  = threadIdx.x;
-  const int lane = tid & 63, w = tid >> 6;
-  // wave 0: diagonal block column `lane`; wave 1: row-panel columns
-  const int c    = (w == 0) ? kb + lane : kb + CH_NB + blockIdx.x * RP_EXTRA + (w - 1) * 64 + lane;
-  const bool act = c < np;
-  const int cc   = act ? c : kb;
-
-  if (*info != 0)
-    return;
-
-  double a[CH_NB];
-  double rdl = 0.0;   // wave 0, lane j: 1 / u_jj
-  int fail   = 0;
-
-#pragma unroll
-  for (int r = 0; r < CH_NB; ++r)
-    a[r] = (w > 0 || r <= lane) ? S[(size_t) (kb + r) * np + cc] : 0.0;
-
-#pragma unroll
-  for (int j = 0; j < CH_NB; ++j)
-  {
-    const int bsel = j & 1;
-
-    if (w == 0)
-    {
-      const double dn = bcast_lane (a[j], j);
-
-      fail = (fail == 0 && !(dn > 0.0)) ? j + 1 : fail;
-
-      const double un = sqrt (dn);
-      const double rn = 1.0 / un;
-
-      a[j]          = (lane == j) ? un : a[j] * rn;
-      R[bsel][lane] = a[j];
-      rdl           = (lane == j) ? rn : rdl;
-
-      if (lane == j)
-        Rr[bsel] = rn;
-    }
-
-    __syncthreads ();
-
-    const double rn = Rr[bsel];
-
-    if (w > 0)
-      a[j] = a[j] * rn;
-
-    double rr[CH_NB];
-
-#pragma unroll
-    for (int r = j + 1; r < CH_NB; ++r)
-      rr[r] = R[bsel][r];
-
-    const double uj = a[j];
-
-#pragma unroll
-    for (int r = j + 1; r < CH_NB; ++r)
-      a[r] = fma (-rr[r], uj, a[r]);
-  }
-
-  if (tid == 0)
-    s_fail = fail;
-
-  __syncthreads ();
-
-  if (s_fail != 0)
-  {
-    if (blockIdx.x == 0 && tid == 0)
-      *info = kb + s_fail;
-
-    return;
-  }
-
-  if (w == 0)
-  {
-    if (blockIdx.x == 0)
-    {
-#pragma unroll
-      for (int r = 0; r < CH_NB; ++r)
-        if (r <= lane)
-          Ud[r * CH_NB + lane] = a[r];
-
-      rd[lane] = rdl;
-    }
-  }
-  else if (act)
-  {
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r)
-      S[(size_t) (kb + r) * np + c] = a[r];
-  }
-}
-
-// the factored diagonal blocks (upper triangles) into S
-__global__ void __launch_bounds__ (256)
-k_copy_diag (double *__restrict__ S, int np, const double *__restrict__ diagbuf)
-{
-  const int kb = blockIdx.x * CH_NB;
-  const int nb = (np - kb < CH_NB) ? np - kb : CH_NB;
-  const double *D = diagbuf + (size_t) blockIdx.x * CH_NB * CH_NB;
-
-  for (int e = threadIdx.x; e < CH_NB * CH_NB; e += 256)
-  {
-    const int r = e >> 6, c = e & 63;
-
-    if (r < nb && c < nb && c >= r)
-      S[(size_t) (kb + r) * np + kb + c] = D[e];
-  }
 }
 
 // lower triangle <- transpose of the upper factor (for the backward solve)
@@ -1066,15 +723,12 @@ k_mirror_lower (double *__restrict__ S, int np)
     S[(size_t) r * np + c] = S[(size_t) c * np + r];
 }
 
-constexpr int SP_NB  = 4 * CH_NB;   // super-panel: four panels
-constexpr int SP_MIN = 4096;        // columns left above which super-panels are used
-
 // S[off:][off:] -= (rank-K product of the rows kb .. kb+K), upper triangle:
 // 128-wide tiles while they number at least 16384 (trailing size above
 // about 23000: more reuse per staged operand), 64-wide ones below (measured
 // faster at n = 20000 and below)
-static void
-trailing_update (double *S, int np, int K, int off, int kb, hipStream_t s)
+hipError_t
+launch_trailing_update (double *S, int np, int K, int off, int kb, hipStream_t s)
 {
   const int nt128 = (np - off + 127) / 128;
 
@@ -1082,83 +736,8 @@ trailing_update (double *S, int np, int K, int off, int kb, hipStream_t s)
     launch_syrk_mfma<1, 128> (S, np, K, np, off, kb, S, s);
   else
     launch_syrk_mfma<1, 64> (S, np, K, np, off, kb, S, s);
-}
-
-// Right-looking blocked Cholesky S = U^T U in 64-row panels: per panel, the
-// row-panel factorisation (diagonal factor and row-panel solve in one
-// launch), then the FP64-MFMA trailing update of the upper triangle; in a
-// super-panel, each panel's update is applied to the super-panel's own rows
-// only, and the rest of the trailing matrix gets one rank-256 update.  Factored diagonal blocks wait in
-// diagbuf until the end; *info is the 1-based failing pivot, 0 on success.
-hipError_t
-launch_potrf (double *S, int np, int *info, double *diagbuf, hipStream_t s)
-{
-  const int npan = (np + CH_NB - 1) / CH_NB;
-  double *rdall  = diagbuf + (size_t) npan * CH_NB * CH_NB;
-
-  for (int kb = 0; kb < np;)
-  {
-    // while more than SP_MIN columns remain: super-panels of four full
-    // panels, whose trailing update is one rank-256 product instead of four
-    // rank-64 ones (a 4x shorter stream over the trailing matrix: 12000
-    // columns factor in 18.7 ms against 25.3 ms); below that the per-panel
-    // steps are as fast or faster
-    if (np - kb > SP_MIN)
-    {
-      const int ke = kb + SP_NB;
-
-      for (int kp = kb; kp < ke; kp += CH_NB)
-      {
-        const int rest = np - kp - CH_NB;
-        const int gr   = (rest + RP_EXTRA - 1) / RP_EXTRA;
-
-        hipLaunchKernelGGL (k_potrf_rowpanel, dim3 (gr), dim3 (64 + RP_EXTRA), 0, s, S, np, kp, info,
-                            diagbuf + (size_t) (kp / CH_NB) * CH_NB * CH_NB, rdall + kp);
-
-        // the rank-64 update of the super-panel's own rows below this panel
-        if (kp + CH_NB < ke)
-          launch_syrk_mfma<1, 64> (S, np, CH_NB, np, kp + CH_NB, kp, S, s, ke);
-      }
-
-      trailing_update (S, np, SP_NB, ke, kb, s);
-      kb = ke;
-      continue;
-    }
-
-    const int nb   = (np - kb < CH_NB) ? np - kb : CH_NB;
-    const int rest = np - kb - nb;
-    double *db     = diagbuf + (size_t) (kb / CH_NB) * CH_NB * CH_NB;
-
-    if (nb == CH_NB)
-    {
-      const int gr = (rest + RP_EXTRA - 1) / RP_EXTRA;
-
-      hipLaunchKernelGGL (k_potrf_rowpanel, dim3 (gr > 0 ? gr : 1), dim3 (64 + RP_EXTRA), 0, s, S, np, kb, info, db,
-                          rdall + kb);
-    }
-    else
-    {
-      hipLaunchKernelGGL (k_potrf_panel, dim3 ((rest > 0) ? (rest + 63) / 64 : 1), dim3 (256), 0, s, S, np, kb, nb,
-                          info, db);
-    }
-
-    if (rest > 0)
-      trailing_update (S, np, nb, kb + nb, kb, s);
-
-    kb += nb;
-  }
-
-  hipLaunchKernelGGL (k_copy_diag, dim3 ((np + CH_NB - 1) / CH_NB), dim3 (256), 0, s, S, np, diagbuf);
-  hipLaunchKernelGGL (k_mirror_lower, dim3 ((np + 255) / 256, np), dim3 (256), 0, s, S, np);
 
   return hipGetLastError ();
-}
-
-size_t
-potrf_diag_doubles (int np)
-{
-  // the factored diagonal blocks, then the reciprocals of their diagonals
-  return (size_t) ((np + CH_NB - 1) / CH_NB) * CH_NB * CH_NB + (size_t) np + CH_NB;
 }
 
 // U^T y = b then U x = y with the factor of launch_potrf (upper triangle =
@@ -1331,8 +910,9 @@ launch_trsv_backward (const double *S, int np, double *y, double *x, hipStream_t
   return hipGetLastError ();
 }
 
-// The same two sweeps as one launch each, chained by flags: one 64-lane
-// block per panel, block k taking the k-th panel in sweep order.  A block
+// The backward sweep as one launch, chained by flags: one 64-lane block per
+// panel, block k taking the k-th panel in sweep order (the forward sweep runs
+// inside the factorisation, k_potrf.hip).  A block
 // applies the contributions of the panels before it in sweep order, each
 // as soon as that panel's flag carries this call's epoch, with the order
 // and arithmetic of k_trsv_panel (the solution is the same to the bit),
@@ -1341,9 +921,8 @@ launch_trsv_backward (const double *S, int np, double *y, double *x, hipStream_t
 // flag is awaited.  The host launches the chain only when every block of
 // the grid can be resident at once, so each wait ends; a wait longer than
 // spin_limit polls still ends the kernel, with *status = epoch (no later
-// block of either sweep does anything then), and the host solves again with
+// block does anything then), and the host solves again with
 // the panel launches.
-template <int FWD>
 __global__ void __launch_bounds__ (64)
 k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ rhs, double *__restrict__ out,
               unsigned *__restrict__ flags, unsigned epoch, unsigned spin_limit, unsigned *__restrict__ status)
@@ -1354,7 +933,7 @@ k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ r
   const int lane = threadIdx.x;
   const int npan = (np + TS_NB - 1) / TS_NB;
   const int k    = blockIdx.x;
-  const int pan  = FWD ? k : npan - 1 - k;
+  const int pan  = npan - 1 - k;
   const int p0   = pan * TS_NB;
   const int pb   = (np - p0 < TS_NB) ? np - p0 : TS_NB;
 
@@ -1373,7 +952,7 @@ k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ r
 
   for (int kk = 0; kk < k; ++kk)
   {
-    const int q  = FWD ? kk : npan - 1 - kk;
+    const int q  = npan - 1 - kk;
     const int q0 = q * TS_NB;
     const int qb = (np - q0 < TS_NB) ? np - q0 : TS_NB;
     double v[TS_NB];
@@ -1439,12 +1018,12 @@ k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ r
 
 #pragma unroll
     for (int j = 0; j < TS_NB; ++j)
-      t[j] = (FWD ? (j < i) : (j > i)) ? T[i][j] : 0.0;
+      t[j] = (j > i) ? T[i][j] : 0.0;
 
 #pragma unroll
     for (int step = 0; step < TS_NB; ++step)
     {
-      const int j     = FWD ? step : TS_NB - 1 - step;
+      const int j     = TS_NB - 1 - step;
       const double yj = bcast_lane (bi * rdl, j);
 
       bi = (i == j) ? yj : fma (-t[j], yj, bi);
@@ -1454,13 +1033,13 @@ k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ r
   {
     for (int step = 0; step < pb; ++step)
     {
-      const int j     = FWD ? step : pb - 1 - step;
+      const int j     = pb - 1 - step;
       const double bj = bcast_lane (bi, j);
       const double yj = bj * rdiag[j];
 
       if (i == j)
         bi = yj;
-      else if (FWD ? (i > j) : (i < j))
+      else if (i < j)
         bi = fma (-T[i][j], yj, bi);
     }
   }
@@ -1484,28 +1063,20 @@ trsv_chain_max_panels ()
 
     (void) hipGetDevice (&dev);
     (void) hipDeviceGetAttribute (&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb, k_trsv_chain<1>, 64, 0);
-
-    int nb0 = 0;
-
-    (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb0, k_trsv_chain<0>, 64, 0);
-    nb  = (nb0 < nb) ? nb0 : nb;
+    (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb, k_trsv_chain, 64, 0);
     cap = (nb > 0 && ncu > 0) ? nb * ncu : 0;
   }
 
   return cap;
 }
 
-// flags: status word, then 2 npan panel flags (forward, backward)
+// flags: status word, then npan panel flags
 hipError_t
-launch_trsv_chain (const double *S, int np, double *b, double *tmp, unsigned *flags, unsigned epoch, hipStream_t s)
+launch_trsv_chain (const double *S, int np, const double *y, double *x, unsigned *flags, unsigned epoch, hipStream_t s)
 {
   const int npan = (np + TS_NB - 1) / TS_NB;
 
-  hipLaunchKernelGGL (k_trsv_chain<1>, dim3 (npan), dim3 (64), 0, s, S, np, b, tmp, flags + 1, epoch, 1u << 22,
-                      flags);
-  hipLaunchKernelGGL (k_trsv_chain<0>, dim3 (npan), dim3 (64), 0, s, S, np, tmp, b, flags + 1 + npan, epoch,
-                      1u << 22, flags);
+  hipLaunchKernelGGL (k_trsv_chain, dim3 (npan), dim3 (64), 0, s, S, np, y, x, flags + 1, epoch, 1u << 22, flags);
 
   return hipGetLastError ();
 }

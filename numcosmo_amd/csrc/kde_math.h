@@ -11,12 +11,17 @@ namespace nck
 // and one third-order step.  With e = 1 - u r^2 the exact value is
 // r (1 - e)^{-1/2} = r (1 + e / 2 + 3 e^2 / 8 + O(e^3)), and e^3 is below 2^-66.
 __device__ inline double
-rsqrt_f64 (double u)
+rsqrt_step (double u, double r)
 {
-  const double r = __builtin_amdgcn_rsq (u);
   const double e = fma (-(u * r), r, 1.0);
 
   return fma (r * e, fma (0.375, e, 0.5), r);
+}
+
+__device__ inline double
+rsqrt_f64 (double u)
+{
+  return rsqrt_step (u, __builtin_amdgcn_rsq (u));
 }
 
 // u^{-p/2} for u >= 1 and a wave-uniform p in [1, 127]: the p-th power of

@@ -298,14 +298,16 @@ hipError_t launch_residual (const double *AT, int nk, int nobs, const double *x,
 hipError_t launch_gather_sym (const double *M, int n, const int *P, int np, double *S,
                               const double *b, double *bs, hipStream_t s);
 size_t potrf_diag_doubles (int np);
-hipError_t launch_potrf (double *S, int np, int *info, double *diagbuf, hipStream_t s);
+// S = U^T U with b replaced by U^{-T} b (k_potrf.hip)
+hipError_t launch_potrf (double *S, int np, double *b, int *info, double *diagbuf, hipStream_t s);
+hipError_t launch_trailing_update (double *S, int np, int K, int off, int kb, hipStream_t s);
 hipError_t launch_trsv_pair (const double *S, int np, double *b, double *tmp, hipStream_t s);
-// the same solve as two flag-chained launches (np / 64 panels at most
-// trsv_chain_max_panels ()); flags holds 1 + 2 ceil(np / 64) words, zero or
+// the backward sweep U x = y as one flag-chained launch (np / 64 panels at
+// most trsv_chain_max_panels ()); flags holds 1 + ceil(np / 64) words, zero or
 // from earlier epochs; flags[0] == epoch afterwards means the chain gave up
-// and b is not the solution
+// and x is not the solution
 int trsv_chain_max_panels ();
-hipError_t launch_trsv_chain (const double *S, int np, double *b, double *tmp, unsigned *flags, unsigned epoch,
+hipError_t launch_trsv_chain (const double *S, int np, const double *y, double *x, unsigned *flags, unsigned epoch,
                               hipStream_t s);
 hipError_t launch_lu_solve (double *S, int np, double *b, int *info, hipStream_t s);
 hipError_t launch_trsv_backward (const double *S, int np, double *y, double *x, hipStream_t s);
