@@ -8,26 +8,40 @@
 // queries, never from reassociating a sum.
 #include "nckde_internal.h"
 
+#include <algorithm>
+
 #pragma clang fp contract(off)
 
 namespace nck
 {
 
 // --------------------------------------------------------------------------
-// NcmStatsVec covariance (ncm_stats_vec.c:510-565, :2376-2399).  One thread
-// per (a <= b) entry follows the one-pass West/Welford recurrence over the
-// rows in their insertion order; the per-entry recurrence needs only the
-// running means of columns a and b, which the thread tracks itself.
+// NcmStatsVec covariance (ncm_stats_vec.c:510-565, :2376-2399): the one-pass
+// West/Welford recurrence over the rows in their insertion order, per entry
+// with the reference's operations.
+//
+// With w = 1, the step of entry (a, b) from row t is
+//   acc += (x_a - mean_a(t)) (x_b - mean_b(t - 1)),
+// and only the means are a long recurrence: once a row's n_a = x_a - mean_a(t)
+// and o_b = x_b - mean_b(t - 1) are known, an entry's chain is one addition.
+// So wave 0 of a block runs the means, one column per lane (with the diagonal
+// entries, t delta R), and leaves n and o in LDS; the other waves form the
+// products of the chunk before.  The bound is wave 0's chain of five FP64
+// operations per row (about 30 cycles each) for one long matrix, and the LDS
+// reads of the products for many short ones.  An entry per thread with its own
+// two means took 15 operations per row and entry: d = 32, n = 10000, k = 500
+// 4.6 -> 2.0 ms for the global and the local matrices, d = 16, n = 3200 0.47 ->
+// 0.28 ms, d = 64, n = 20000, k = 1000 25.4 -> 16.9 ms.
 //
 // The division R = delta / W_t (W_t = t + 1, the weight after row t) sits on
-// the recurrence's critical path.  The reciprocals y_t = RN(1 / W_t) are
-// formed beside each staged chunk, off that path, and the quotient is
-// rebuilt from them: q = RN(delta y_t), r = delta - q W_t (exact in an FMA),
-// RN(q + r y_t), which is the correctly rounded delta / W_t for a faithful q
-// and a correctly rounded y_t (Markstein's theorem); r = 0 keeps q, and with
-// it the sign of a zero quotient.
+// the chain.  The reciprocals y_t = RN(1 / W_t) are formed with each staged
+// chunk, and the quotient is rebuilt from them: q = RN(delta y_t), r = delta -
+// q W_t (exact in an FMA), RN(q + r y_t), which is the correctly rounded
+// delta / W_t for a faithful q and a correctly rounded y_t (Markstein's
+// theorem; a zero quotient may change its sign, which no sum here can see).
 // --------------------------------------------------------------------------
-constexpr int WF_LDS = 4096;   // doubles of LDS per block: 4096 / d rows staged per step
+constexpr int WF_CHUNK = 2048;  // entries (rows x columns) of a staged chunk, at most
+constexpr int WF_STAGE = 8;     // of them per staging thread
 
 __device__ inline double
 div_by_recip (double a, double b, double y)
@@ -35,161 +49,241 @@ div_by_recip (double a, double b, double y)
   const double q = a * y;
   const double r = fma (-q, b, a);
 
-  return (r == 0.0) ? q : fma (r, y, q);
+  return fma (r, y, q);
 }
 
-// Thread p of a matrix: the diagonal entries (p < d) take the first d
-// threads, the off-diagonal pairs a < b start at the next multiple of 64, so
-// that no wave runs both recurrences.
-__device__ inline bool
-welford_pair (int p, int d, int &a, int &b)
+// first row and column of 2 x 2 tile q of the upper triangle
+__device__ inline void
+welford_tile (int q, int d, int &a, int &b)
 {
-  const int dpad = (d + 63) & ~63;
+  const int nt = (d + 1) / 2;
+  int ta       = 0;
 
-  if (p < d)
+  while (q >= nt - ta)
   {
-    a = b = p;
-    return true;
+    q -= nt - ta;
+    ++ta;
   }
 
-  int q = p - dpad;
-
-  if (q < 0 || q >= d * (d - 1) / 2)
-    return false;
-
-  a = 0;
-
-  while (q >= d - 1 - a)
-  {
-    q -= d - 1 - a;
-    ++a;
-  }
-
-  b = a + 1 + q;
-
-  return true;
+  a = 2 * ta;
+  b = 2 * (ta + q);
 }
 
-__global__ void __launch_bounds__ (256)
-k_welford_cov (const double *__restrict__ X, int d, int nrows, const int *__restrict__ rows,
-               int rows_stride, int nmats, double *__restrict__ cov_out)
+// A product thread holds a 2 x 2 tile of entries (one per thread: 136 tiles at
+// d = 32, 528 at d = 64), which halves the LDS reads per entry.
+__global__ void __launch_bounds__ (640)
+k_welford_cov (const double *__restrict__ X, int d, int nrows, const int *__restrict__ rows, int rows_stride,
+               int rc, double *__restrict__ cov_out)
 {
-  extern __shared__ double xs[];   // (WF_LDS / d) rows x d, then their reciprocal weights
-  const long mat   = blockIdx.y + (long) blockIdx.z * gridDim.y;
-  const int p      = blockIdx.x * blockDim.x + threadIdx.x;
+  extern __shared__ double lds[];          // rc rows per chunk
+  const long mat   = blockIdx.x;
+  const int csz    = rc * d;
+  double *xo       = lds;                  // 3 chunks: x, then o = x - mean(t - 1) in its place
+  double *nn       = lds + 3 * csz;        // 2 chunks: n = x - mean(t)
+  double *yr       = nn + 2 * csz;         // 3 chunks of reciprocals
+  const int lane   = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int st     = threadIdx.x - 64;     // staging and product thread
+  const int nst    = blockDim.x - 64;
+  const int *rw    = rows ? rows + mat * (size_t) rows_stride : nullptr;
+  const int ntile  = ((d + 1) / 2) * ((d + 1) / 2 + 1) / 2;
+  const int nchunk = (nrows + rc - 1) / rc;
+  int pa = 0, pb = 0;
+  double acc[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
+  int se[WF_STAGE], sr[WF_STAGE];          // column and row in the chunk of this thread's staged entries
 
-  if (mat >= nmats)
-    return;
-
-  int a = 0, b = 0;
-  const bool active = welford_pair (p, d, a, b);
-
-  const int *rw  = rows ? rows + mat * (size_t) rows_stride : nullptr;
-  const double w = 1.0;
-  double mean_a = 0.0, mean_b = 0.0, acc = 0.0, weight = 0.0, weight2 = 0.0;
-
-  const int chunk = WF_LDS / d;
-
-  for (int t0 = 0; t0 < nrows; t0 += chunk)
+  if (w > 0)
   {
-    const int cnt = (nrows - t0 < chunk) ? nrows - t0 : chunk;
-
-    double *rc = xs + chunk * d;
-
-    for (int e = threadIdx.x; e < cnt * d; e += blockDim.x)
-    {
-      const int t    = e / d, col = e - t * d;
-      const size_t r = rw ? (size_t) rw[t0 + t] : (size_t) (t0 + t);
-
-      xs[e] = X[r * d + col];
-    }
-
-    for (int t = threadIdx.x; t < cnt; t += blockDim.x)
-      rc[t] = 1.0 / (double) (t0 + t + 1);
-
-    __syncthreads ();
-
-    // one row of the recurrence
-    auto step = [&] (double xa, double xb, double y) {
-      const double curweight = weight + w;
-      const double delta_a   = xa - mean_a;
-      const double R_a       = div_by_recip (delta_a * w, curweight, y);
-
-      if (a == b)
-      {
-        const double dvar = weight * delta_a * R_a;
-
-        acc    = acc + dvar;
-        mean_a = mean_a + R_a;
-      }
-      else
-      {
-        const double mean_a_new = mean_a + R_a;
-        const double dC         = w * (xa - mean_a_new) * (xb - mean_b);
-        const double delta_b    = xb - mean_b;
-        const double R_b        = div_by_recip (delta_b * w, curweight, y);
-
-        acc    = acc + dC;
-        mean_a = mean_a_new;
-        mean_b = mean_b + R_b;
-      }
-
-      weight  = curweight;
-      weight2 = weight2 + w * w;
-    };
-
-    if (active)
-    {
-      // rows four at a time, their LDS reads issued before the recurrence
-      int t = 0;
-
-      for (; t + 4 <= cnt; t += 4)
-      {
-        double xa[4], xb[4], y[4];
+    if (st < ntile)
+      welford_tile (st, d, pa, pb);
 
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < WF_STAGE; ++u)
+    {
+      const int e = st + u * nst;
+
+      sr[u] = e / d;
+      se[u] = e - sr[u] * d;
+    }
+  }
+
+  // chunk c from global memory to xo[c % 3]
+  auto stage_in = [&] (int c, double (&v)[WF_STAGE]) {
+    const int cnt = min (rc, nrows - c * rc);
+
+#pragma unroll
+    for (int u = 0; u < WF_STAGE; ++u)
+    {
+      v[u] = 0.0;
+
+      if (sr[u] < cnt)
+      {
+        const size_t r = rw ? (size_t) rw[c * rc + sr[u]] : (size_t) (c * rc + sr[u]);
+
+        v[u] = X[r * d + se[u]];
+      }
+    }
+  };
+  auto stage_out = [&] (int c, const double (&v)[WF_STAGE]) {
+    const int cnt = min (rc, nrows - c * rc);
+    double *to    = xo + (c % 3) * csz;
+
+#pragma unroll
+    for (int u = 0; u < WF_STAGE; ++u)
+      if (sr[u] < cnt)
+        to[sr[u] * d + se[u]] = v[u];
+
+    for (int t = st; t < cnt; t += nst)
+      yr[(c % 3) * rc + t] = 1.0 / (double) (c * rc + t + 1);
+  };
+
+  double mean = 0.0, var = 0.0, W = 0.0;
+  double v[WF_STAGE];
+
+  if (w > 0)
+  {
+    stage_in (0, v);
+    stage_out (0, v);
+  }
+
+  __syncthreads ();
+
+  for (int c = 0; c <= nchunk; ++c)
+  {
+    if (w == 0)
+    {
+      if (c < nchunk && lane < d)
+      {
+        const int cnt   = min (rc, nrows - c * rc);
+        double *xc      = xo + (c % 3) * csz + lane;
+        double *nc      = nn + (c & 1) * csz + lane;
+        const double *y = yr + (c % 3) * rc;
+
+        auto step = [&] (int t, double x, double yt) {
+          const double Wn    = W + 1.0;
+          const double delta = x - mean;
+          const double R     = div_by_recip (delta, Wn, yt);
+
+          mean      = mean + R;
+          var       = var + W * delta * R;
+          W         = Wn;
+          xc[t * d] = delta;
+          nc[t * d] = x - mean;
+        };
+        int t = 0;
+
+        // rows four at a time, their LDS reads issued before the recurrence
+        for (; t + 4 <= cnt; t += 4)
         {
-          xa[u] = xs[(t + u) * d + a];
-          xb[u] = xs[(t + u) * d + b];
-          y[u]  = rc[t + u];
+          double x[4], yt[4];
+
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+          {
+            x[u]  = xc[(t + u) * d];
+            yt[u] = y[t + u];
+          }
+
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            step (t + u, x[u], yt[u]);
         }
 
+        for (; t < cnt; ++t)
+          step (t, xc[t * d], y[t]);
+      }
+    }
+    else
+    {
+      if (c + 1 < nchunk)
+        stage_in (c + 1, v);
+
+      if (c > 0 && st < ntile)
+      {
+        const int cnt   = min (rc, nrows - (c - 1) * rc);
+        const double *o = xo + ((c - 1) % 3) * csz + pb;
+        const double *n = nn + ((c - 1) & 1) * csz + pa;
+        int t           = 0;
+
+        // (column d of an odd d is the next row's first entry: not used)
+        for (; t + 4 <= cnt; t += 4)
+        {
+          double p[4][2][2];
+
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-          step (xa[u], xb[u], y[u]);
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                p[q][i][j] = n[(t + q) * d + i] * o[(t + q) * d + j];
+
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[i][j] = acc[i][j] + p[q][i][j];
+        }
+
+        for (; t < cnt; ++t)
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+              acc[i][j] = acc[i][j] + n[t * d + i] * o[t * d + j];
       }
 
-      for (; t < cnt; ++t)
-        step (xs[t * d + a], xs[t * d + b], rc[t]);
+      if (c + 1 < nchunk)
+        stage_out (c + 1, v);
     }
 
     __syncthreads ();
   }
 
-  if (active)
-  {
-    const double bias_wt = 1.0 / (weight - weight2 / weight);
-    double *C            = cov_out + mat * (size_t) d * d;
-    const double v       = acc * bias_wt;
+  const double weight  = (double) nrows;
+  const double bias_wt = 1.0 / (weight - weight / weight);
+  double *C            = cov_out + mat * (size_t) d * d;
 
-    C[a * d + b] = v;
-    C[b * d + a] = v;
+  if (w == 0)
+  {
+    if (lane < d)
+      C[lane * d + lane] = var * bias_wt;
+
+    return;
   }
+
+  if (st < ntile)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (pa + i < pb + j && pb + j < d)
+        {
+          const double val = acc[i][j] * bias_wt;
+
+          C[(pa + i) * d + pb + j] = val;
+          C[(pb + j) * d + pa + i] = val;
+        }
 }
 
 hipError_t
 launch_welford_cov (const double *X, int d, int nrows, const int *rows, int rows_stride, int nmats,
                     double *cov, hipStream_t s)
 {
-  const int nthr   = ((d + 63) & ~63) + d * (d - 1) / 2;
-  const int bs     = 256;
-  const int gy     = nmats < 32768 ? nmats : 32768;
-  const int gz     = (nmats + gy - 1) / gy;
-  dim3 grid ((nthr + bs - 1) / bs, gy, gz);
+  const int ntile = ((d + 1) / 2) * ((d + 1) / 2 + 1) / 2;
 
-  hipLaunchKernelGGL (k_welford_cov, grid, dim3 (bs), sizeof (double) * ((WF_LDS / d) * d + WF_LDS / d), s, X, d,
-                      nrows, rows, rows_stride, nmats, cov);
+  // a single matrix: four staging waves at least, so that a chunk is long
+  // against the latency of its loads
+  const int nw = std::max ((ntile + 63) / 64, (nmats < 64) ? 4 : 1);
+  const int rc = std::min (WF_CHUNK, 64 * nw * WF_STAGE) / d;
+
+  // two chunks of n, three of o and of the reciprocals, one column past the end
+  const size_t lds = sizeof (double) * (5 * (size_t) rc * d + 3 * (size_t) rc + 2);
+
+  if (nmats > 0)
+    hipLaunchKernelGGL (k_welford_cov, dim3 (nmats), dim3 (64 + 64 * nw), lds, s, X, d, nrows, rows, rows_stride, rc,
+                        cov);
 
   return hipGetLastError ();
 }
