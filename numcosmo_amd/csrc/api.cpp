@@ -1321,7 +1321,7 @@ ensure_mixed (nckde *h)
 {
   const int d   = h->d;
   const int DP  = nck::mfma_dim (d);
-  const int kpt = (DP >= 32) ? 1 : 32 / DP;
+  const int kpt = nck::mixed_group (DP);
   const size_t n_pad = ((h->n_k + kpt - 1) / kpt) * kpt;
 
   if (!h->mixed_ready)
@@ -1399,8 +1399,8 @@ ensure_f32 (nckde *h)
 // the padded dimension D otherwise), log2 n and log2 m of the tuned case,
 // split count.  An eval uses the entry of its precision and dimension
 // nearest in (log2 n, log2 m) within one octave in each, else the default
-// rule: about 8192 blocks in all and at least 8 kernel groups per split
-// (mixed), about 16384 blocks and at least 32 kernels per split (FP64 and
+// rule: about 8192 blocks in all and at least 8 (DP >= 32) or 256 / DP kernels
+// per split (mixed), about 16384 blocks and at least 32 kernels per split (FP64 and
 // FP32).  Many short splits keep a split's kernel factors in its XCD's L2
 // and even out the blocks' finishing times.
 struct SplitTune
@@ -1442,8 +1442,9 @@ static int
 mixed_nsplit (const nckde *h, size_t m)
 {
   const int DP      = nck::mfma_dim (h->d);
-  const int kpt     = (DP >= 32) ? 1 : 32 / DP;
+  const int kpt     = nck::mixed_group (DP);
   const int ngroups = (int) ((h->n_k + kpt - 1) / kpt);
+  const int kmin    = (DP >= 32) ? 8 : 256 / DP;   // kernels per split, at least (default rule)
   int chosen        = (h->split_override > 0) ? (int) h->split_override : tuned_nsplit (1, DP, h->n_k, m);
 
   if (chosen > 0)
@@ -1452,7 +1453,7 @@ mixed_nsplit (const nckde *h, size_t m)
   const int bx = (int) ((m + nck::mixed_points_per_block (DP) - 1) / nck::mixed_points_per_block (DP));
   int nsplit   = (8192 + bx - 1) / bx;
 
-  return std::max (1, std::min (nsplit, std::max (1, ngroups / 8)));
+  return std::max (1, std::min (nsplit, (int) (h->n_k / kmin)));
 }
 
 static int

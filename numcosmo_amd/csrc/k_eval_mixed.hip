@@ -37,13 +37,21 @@ typedef float floatx16 __attribute__ ((ext_vector_type (16)));
 constexpr double LOG2E = 1.4426950408889634073599246810018921;
 constexpr double LN2   = 0.69314718055994530941723212145817657;
 
+// rows of a kernel per 32-row MFMA tile
+constexpr int
+mixed_rows (int DP)
+{
+  return (DP == 4) ? 4 : (DP <= 16) ? 8 : 16;
+}
+
 template <int DP>
 struct Plan
 {
-  static constexpr int KPT    = (DP >= 32) ? 1 : 32 / DP;  // kernels per 32-row tile
-  static constexpr int NRT    = (DP == 64) ? 2 : 1;        // row tiles per kernel group
+  static constexpr int RG     = mixed_rows (DP);           // rows of a kernel in one 32-row tile
+  static constexpr int KPT    = mixed_group (DP);          // kernels per group
+  static constexpr int NRG    = DP / RG;                   // row tiles per group
   static constexpr int NKB    = (DP >= 32) ? DP / 16 : 1;  // 16-wide K blocks
-  static constexpr int NLOCAL = (DP == 4) ? 4 : (DP == 8 ? 2 : 1);   // kernels per lane
+  static constexpr int NLOCAL = 16 / RG;                   // kernels per lane
 };
 
 int
@@ -371,111 +379,95 @@ k_colmean (const double *__restrict__ X, int n, int d, double *__restrict__ mu)
 // each lane adds a 32-bit offset, so the loads take the scalar-base form and
 // need no 64-bit vector address arithmetic.
 //
-// Row map of a 32-row tile.  The 32x32 accumulator gives lane l the rows
-// 8 j + 4 (l / 32) + r (j, r < 4).  Kernel rows are placed so that these
-// rows hold whole kernels and no lane needs a partner's partial sum:
-//   DP = 4:  row R = kernel R / 4, dim R % 4 (kernels 2 j + g);
-//   DP = 8:  row 8 j + 4 g + r = kernel 2 g + j / 2, dim 4 (j % 2) + r;
-//   DP = 16: row 8 j + 4 g + r = kernel g, dim 4 j + r.
-// At DP >= 32 one kernel fills the tile and the half-waves add partials.
+// Row tiles.  A group is 32 / RG kernels; row tile rg holds the rows rg RG ..
+// rg RG + RG - 1 of all of them, because A_i is lower triangular (the product
+// of two such factors): these rows need only their first (rg + 1) RG columns.
+// The split product of a row over K columns takes 3 K slots, so with RG = 16
+// a tile takes 3 (rg + 1) MFMAs (9 for a pair of kernels at DP = 32, 30 at DP =
+// 64, where whole kernels took 12 and 48); with RG = 8 at DP = 16 the upper tile
+// packs its 8 + 8 + 8 slots in two (5 for four kernels, 6 before).  At DP = 8
+// the same with RG = 4 saves a quarter of the MFMAs but costs registers, and
+// the vector work bounds it: 289 against 275 us (n = 4000, m = 100000).
+//
+// Row map of a tile.  The 32x32 accumulator gives lane l the rows 8 j + 4 (l /
+// 32) + r (j, r < 4).  Kernel rows are placed so that these rows hold whole
+// row groups and no lane needs a partner's partial sum:
+//   RG = 4:  row R = kernel R / 4, dim R % 4 (kernels 2 j + g);
+//   RG = 8:  row 8 j + 4 g + r = kernel 2 g + j / 2, dim 4 (j % 2) + r;
+//   RG = 16: row 8 j + 4 g + r = kernel g, dim 4 j + r.
 template <int DP>
 __device__ inline void
 tile_row (unsigned R, unsigned &kl, unsigned &dim)
 {
-  if (DP == 4)
+  if (Plan<DP>::RG == 4)
   {
     kl  = R >> 2;
     dim = R & 3;
   }
-  else if (DP == 8)
+  else if (Plan<DP>::RG == 8)
   {
     kl  = 2 * ((R >> 2) & 1) + (R >> 4);
     dim = ((R >> 3) & 1) * 4 + (R & 3);
   }
-  else if (DP == 16)
+  else
   {
     kl  = (R >> 2) & 1;
     dim = (R >> 3) * 4 + (R & 3);
   }
-  else
-  {
-    kl  = 0;
-    dim = R;
-  }
 }
-template <int DP>
+
+// four halves of a row's hi part beside the same four of its lo part
 __device__ inline half8
-load_a_frag (const _Float16 *__restrict__ A, int tg, int rt, int kb, int lohi, int lane)
+load_hi_lo (const _Float16 *hi, int lo)
 {
-  using P            = Plan<DP>;
-  const unsigned g   = lane >> 5;
-  const unsigned R   = lane & 31;
-  const _Float16 *Ag = A + (size_t) tg * P::KPT * 2 * DP * DP;
-  half8 v;
+  const half4 h = *(const half4 *) hi;
+  const half4 l = *(const half4 *) (hi + lo);
 
-  unsigned kl, row;
-
-  tile_row<DP> (R, kl, row);
-
-  if (DP >= 16)
-  {
-    row += (DP == 64) ? rt * 32 : 0;
-    v = *(const half8 *) (Ag + ((kl * 2 + lohi) * DP * DP + row * DP + kb * 16 + g * 8));
-  }
-  else if (DP == 8)
-  {
-    v = *(const half8 *) (Ag + ((kl * 2 + g) * 64 + row * 8));  // g = 0: hi, 1: lo
-  }
-  else
-  {
-    const _Float16 *bh = Ag + (kl * 2 * 16 + row * 4);
-    const half4 h      = *(const half4 *) bh;
-    const half4 l      = *(const half4 *) (bh + 16);
-
-    v = (half8) {h[0], h[1], h[2], h[3], l[0], l[1], l[2], l[3]};
-  }
-
-  return v;
+  return (half8) {h[0], h[1], h[2], h[3], l[0], l[1], l[2], l[3]};
 }
+
+// Point fragments: the hi and lo parts over each K block (DP = 8: all 8 dims
+// in both halves of K), and for packed tiles
+//   DP = 4: hi (0..3) twice | lo (0..3) twice;  DP = 16: hi (0..7) | lo (0..7).
+template <int DP>
+struct PointFrag
+{
+  half8 h[Plan<DP>::NKB], l[Plan<DP>::NKB], p;
+};
 
 template <int DP>
-__device__ inline half8
-load_b_frag (const _Float16 *__restrict__ Yh, const _Float16 *__restrict__ Yl, int p, int kb, int lohi, int lane)
+__device__ inline void
+load_points (PointFrag<DP> &B, const _Float16 *__restrict__ Yh, const _Float16 *__restrict__ Yl, int p, int lane)
 {
-  const int g = lane >> 5;
-  half8 v;
+  const int g          = lane >> 5;
+  const _Float16 *h    = Yh + (size_t) p * DP, *l = Yl + (size_t) p * DP;
+  const _Float16 *mine = g ? l : h;
 
-  if (DP >= 16)
+  if constexpr (DP == 16)
   {
-    const _Float16 *src = (lohi ? Yl : Yh) + (size_t) p * DP + kb * 16 + g * 8;
-
-    v = *(const half8 *) src;
+    B.p = *(const half8 *) mine;
   }
-  else if (DP == 8)
+  else if constexpr (DP == 4)
   {
-    v = *(const half8 *) ((lohi ? Yl : Yh) + (size_t) p * 8);
-  }
-  else
-  {
-    const half4 q = *(const half4 *) ((g ? Yl : Yh) + (size_t) p * 4);
+    const half4 q = *(const half4 *) mine;
 
-    v = (half8) {q[0], q[1], q[2], q[3], q[0], q[1], q[2], q[3]};
+    B.p = (half8) {q[0], q[1], q[2], q[3], q[0], q[1], q[2], q[3]};
   }
 
-  return v;
-}
-
-// Pair reduction across the half-waves with one v_permlane32_swap (it swaps
-// lanes 32-63 of its first operand with lanes 0-31 of its second).  With
-// (a, b) the partial sums of two kernel slots, lanes 0-31 get a[L] + a[L+32]
-// and lanes 32-63 get b[L] + b[L-32]: each half-wave receives the total of
-// the slot it owns.
-__device__ inline float
-halfwave_pair_sum (float a, float b)
-{
-  const auto r = __builtin_amdgcn_permlane32_swap (__float_as_uint (a), __float_as_uint (b), false, false);
-
-  return __uint_as_float (r[0]) + __uint_as_float (r[1]);
+  if constexpr (DP == 8)
+  {
+    B.h[0] = *(const half8 *) h;
+    B.l[0] = *(const half8 *) l;
+  }
+  else if constexpr (DP >= 16)
+  {
+#pragma unroll
+    for (int kb = 0; kb < Plan<DP>::NKB; ++kb)
+    {
+      B.h[kb] = *(const half8 *) (h + kb * 16 + g * 8);
+      B.l[kb] = *(const half8 *) (l + kb * 16 + g * 8);
+    }
+  }
 }
 
 // All lnt2 <= 0: b2_i is taken relative to max_j b_j and the kernel factor is
@@ -505,200 +497,197 @@ lse_push (float c2, float4 cf, float kappa, float M0, float &Mb, float &S32)
   S32 += __builtin_amdgcn_exp2f (lnt);
 }
 
+// The factors of one row tile of a kernel group: A fragments (hi, lo), the
+// (negated) centre terms of the 16 rows held by this lane (8 j + 4 g + r)
 template <int DP>
-struct GroupData
+struct RowData
 {
-  half8 Ah[Plan<DP>::NRT][Plan<DP>::NKB];
-  half8 Al[Plan<DP>::NRT][Plan<DP>::NKB];
-  floatx16 cinit[Plan<DP>::NRT];
-  float4 cf[4];
+  half8 h[Plan<DP>::NKB], l[Plan<DP>::NKB];
+  floatx16 c;
 };
 
 template <int DP>
 __device__ inline void
-load_group (GroupData<DP> &G, const _Float16 *__restrict__ A, const float *__restrict__ cv,
-            const float4 *__restrict__ coef, int tg, int lane)
+load_rows (RowData<DP> &G, const _Float16 *__restrict__ A, const float *__restrict__ cv, int tg, int rg, int lane)
 {
-  using P          = Plan<DP>;
-  const unsigned g = lane >> 5;
-  const float *cg  = cv + (size_t) tg * P::KPT * DP;   // wave-uniform group bases
-  const float4 *fg = coef + (size_t) tg * P::KPT;
+  using P            = Plan<DP>;
+  const unsigned g   = lane >> 5;
+  const _Float16 *Ag = A + (size_t) tg * P::KPT * 2 * DP * DP;   // wave-uniform group bases
+  const float *cg    = cv + (size_t) tg * P::KPT * DP;
+  constexpr int LO   = DP * DP;                                  // lo part after the hi part
+  unsigned kl, dim;
 
-#pragma unroll
-  for (int rt = 0; rt < P::NRT; ++rt)
+  tile_row<DP> (lane & 31, kl, dim);
+
+  const unsigned at = kl * 2 * LO + (rg * P::RG + dim) * DP;
+
+  if constexpr (DP == 4)
+  {
+    G.h[0] = load_hi_lo (Ag + at, LO);
+  }
+  else if constexpr (DP == 8)
+  {
+    G.h[0] = *(const half8 *) (Ag + (at + g * LO));   // hi | lo along K
+  }
+  else
   {
 #pragma unroll
     for (int kb = 0; kb < P::NKB; ++kb)
-    {
-      G.Ah[rt][kb] = load_a_frag<DP> (A, tg, rt, kb, 0, lane);
-
-      if (DP >= 16)
-        G.Al[rt][kb] = load_a_frag<DP> (A, tg, rt, kb, 1, lane);
-    }
-
-    // the (negated) centre terms of the 16 rows held by this lane: rows 8 j + 4 g + r
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-    {
-      unsigned kl, row;
-
-      tile_row<DP> (8 * j + 4 * g, kl, row);
-
-      const float4 c4 = *(const float4 *) (cg + kl * DP + ((DP == 64) ? rt * 32 + row : row));
-
-      G.cinit[rt][4 * j + 0] = c4.x;
-      G.cinit[rt][4 * j + 1] = c4.y;
-      G.cinit[rt][4 * j + 2] = c4.z;
-      G.cinit[rt][4 * j + 3] = c4.w;
-    }
+      if (kb <= rg)
+      {
+        // the packed upper tile of DP = 16 takes its 8 hi columns twice
+        G.h[kb] = *(const half8 *) (Ag + (at + kb * 16 + ((DP == 16 && rg == 0) ? 0 : g * 8)));
+        G.l[kb] = *(const half8 *) (Ag + (at + LO + kb * 16 + g * 8));
+      }
   }
 
-  // coefficients of the kernel slots this lane owns
 #pragma unroll
-  for (int q = 0; q < 4; ++q)
+  for (int j = 0; j < 4; ++j)
   {
-    int slot = 0;
+    unsigned kc, row;
 
-    if (DP == 4)
-      slot = 2 * q + g;
-    else if (DP == 8)
-      slot = 2 * g + (q & 1);
-    else if (DP == 16)
-      slot = g;
+    tile_row<DP> (8 * j + 4 * g, kc, row);
 
-    G.cf[q] = fg[slot];
+    const float4 c4 = *(const float4 *) (cg + kc * DP + rg * P::RG + row);
+
+    G.c[4 * j + 0] = c4.x;
+    G.c[4 * j + 1] = c4.y;
+    G.c[4 * j + 2] = c4.z;
+    G.c[4 * j + 3] = c4.w;
   }
 }
 
-// One kernel group against the NPT point tiles of a wave: all MFMA chains
-// first (separate accumulators), then the VALU reduction and sums, so the
-// matrix cores of tile t+1 overlap the vector work of tile t.
-template <int DP, int KERNEL, int NPT, bool OFFSET, bool SCALED, int NST>
+// coefficients of the kernel slots this lane owns
+template <int DP>
 __device__ inline void
-group_step (const GroupData<DP> &cur, const half8 (&Bh)[NPT][Plan<DP>::NKB], const half8 (&Bl)[NPT][Plan<DP>::NKB],
-            const float (&tscale)[NPT], const float (&it2)[NPT], const float (&M0)[NST], float (&Mb)[NST],
-            float (&S32)[NST], float kappa, int g)
+load_coef (float4 (&cf)[Plan<DP>::NLOCAL], const float4 *__restrict__ coef, int tg, int lane)
 {
-  using P = Plan<DP>;
-  floatx16 acc[NPT][P::NRT];
+  const unsigned g = lane >> 5;
+  const float4 *fg = coef + (size_t) tg * Plan<DP>::KPT;
 
 #pragma unroll
-  for (int t = 0; t < NPT; ++t)
+  for (int q = 0; q < Plan<DP>::NLOCAL; ++q)
+    cf[q] = fg[(Plan<DP>::RG == 4) ? 2 * q + g : (Plan<DP>::RG == 8) ? 2 * g + q : g];
+}
+
+__device__ inline floatx16
+mixed_mfma (half8 a, half8 b, floatx16 c)
+{
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16 (a, b, c, 0, 0, 0);
+}
+
+// z' of one row tile and one point tile: the centre terms plus the split
+// products hi hi + hi lo + lo hi over the tile's columns
+template <int DP, bool SCALED>
+__device__ inline floatx16
+row_product (const RowData<DP> &G, int rg, const PointFrag<DP> &B, float tscale)
+{
+  floatx16 z = G.c;
+
+  if (SCALED)
   {
 #pragma unroll
-    for (int rt = 0; rt < P::NRT; ++rt)
-    {
-      floatx16 c0 = cur.cinit[rt];
-
-      if (SCALED)
-      {
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-          c0[r] *= tscale[t];
-      }
-
-      if (DP == 4)
-      {
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][0], Bh[t][0], c0, 0, 0, 0);
-      }
-      else if (DP == 8)
-      {
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][0], Bh[t][0], c0, 0, 0, 0);
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][0], Bl[t][0], acc[t][rt], 0, 0, 0);
-      }
-      else
-      {
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][0], Bh[t][0], c0, 0, 0, 0);
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][0], Bl[t][0], acc[t][rt], 0, 0, 0);
-        acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Al[rt][0], Bh[t][0], acc[t][rt], 0, 0, 0);
-
-#pragma unroll
-        for (int kb = 1; kb < P::NKB; ++kb)
-        {
-          acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][kb], Bh[t][kb], acc[t][rt], 0, 0, 0);
-          acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Ah[rt][kb], Bl[t][kb], acc[t][rt], 0, 0, 0);
-          acc[t][rt] = __builtin_amdgcn_mfma_f32_32x32x16_f16 (cur.Al[rt][kb], Bh[t][kb], acc[t][rt], 0, 0, 0);
-        }
-      }
-    }
+    for (int r = 0; r < 16; ++r)
+      z[r] *= tscale;
   }
 
-  float tot_prev = 0.0f;
+  if (DP == 4)
+    return mixed_mfma (G.h[0], B.p, z);
+
+  if (DP == 8)
+    return mixed_mfma (G.h[0], B.l[0], mixed_mfma (G.h[0], B.h[0], z));
+
+  // (the lo part's columns 8..15 are zero in the upper tile)
+  if (DP == 16 && rg == 0)
+    return mixed_mfma (G.l[0], B.h[0], mixed_mfma (G.h[0], B.p, z));
 
 #pragma unroll
-  for (int t = 0; t < NPT; ++t)
+  for (int kb = 0; kb < Plan<DP>::NKB; ++kb)
+    if (kb <= rg)
+    {
+      z = mixed_mfma (G.h[kb], B.h[kb], z);
+      z = mixed_mfma (G.h[kb], B.l[kb], z);
+      z = mixed_mfma (G.l[kb], B.h[kb], z);
+    }
+
+  return z;
+}
+
+// One kernel group against the NPT point tiles of a wave.  The tiles' MFMA
+// chains run LAG tiles ahead of the squared norms and kernel sums, so that
+// matrix and vector work overlap within a wave; the fences keep the compiler
+// from grouping all chains first (d = 16, n = 3200, m = 6400: 53 -> 46 us).
+// `next (G, rg)` runs before row tile rg, whose factors are G[rg % NG]: it loads
+// them (NG = 1) or the ones after them (NG = 2).
+template <int DP, int KERNEL, int NPT, bool OFFSET, bool SCALED, int NG, class Next>
+__device__ inline void
+group_step (RowData<DP> (&G)[NG], const float4 (&cf)[Plan<DP>::NLOCAL], const PointFrag<DP> (&B)[NPT],
+            const float (&tscale)[NPT], const float (&it2)[NPT], const float (&M0)[NPT], float (&Mb)[NPT],
+            float (&S32)[NPT], float kappa, const Next &next)
+{
+  using P           = Plan<DP>;
+  constexpr int LAG = (DP >= 16) ? 2 : NPT;   // DP < 16: all chains first (measured equal)
+  constexpr int NQ  = P::NRG * NPT;
+  floatx16 acc[LAG + 1];
+  float part[NPT][P::NLOCAL];
+
+#pragma unroll
+  for (int q = 0; q < NQ + LAG; ++q)
   {
-    // squared norms per kernel slot held by this lane
-    float part[P::NLOCAL];
+    if (q < NQ)
+    {
+      const int rg = q / NPT, t = q % NPT;
 
-#pragma unroll
-    for (int j = 0; j < P::NLOCAL; ++j)
-      part[j] = 0.0f;
+      if (t == 0)
+        next (G, rg);
 
+      acc[q % (LAG + 1)] = row_product<DP, SCALED> (G[rg % NG], rg, B[t], tscale[t]);
+    }
+
+    if (q >= LAG)
+    {
+      const int rg = (q - LAG) / NPT, t = (q - LAG) % NPT;
+      const floatx16 &z = acc[(q - LAG) % (LAG + 1)];
+
+      // squared norms per kernel slot held by this lane, a row tile's rows
+      // summed by themselves (shorter FP32 chains)
 #pragma unroll
-    for (int rt = 0; rt < P::NRT; ++rt)
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
+      for (int j = 0; j < P::NLOCAL; ++j)
       {
-        const int j = (DP == 4) ? r / 4 : ((DP == 8) ? r / 8 : 0);
+        float p = z[j * P::RG] * z[j * P::RG];
 
-        part[j] = fmaf (acc[t][rt][r], acc[t][rt][r], part[j]);
+#pragma unroll
+        for (int r = j * P::RG + 1; r < (j + 1) * P::RG; ++r)
+          p = fmaf (z[r], z[r], p);
+
+        part[t][j] = (rg == 0) ? p : part[t][j] + p;
       }
 
-    const float sc2 = SCALED ? it2[t] : 1.0f;
-
-    if (DP == 4)
-    {
-      // each kernel's 4 rows sit in one lane: slots 2 j + g
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        lse_push<KERNEL, OFFSET> (part[j] * sc2, cur.cf[j], kappa, M0[t], Mb[t], S32[t]);
-    }
-    else if (DP == 8)
-    {
-      // whole kernels per lane: slots 2 g + q
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        lse_push<KERNEL, OFFSET> (part[q] * sc2, cur.cf[q], kappa, M0[t], Mb[t], S32[t]);
-    }
-    else if (DP == 16)
-    {
-      // one whole kernel per lane: slot g
-      lse_push<KERNEL, OFFSET> (part[0] * sc2, cur.cf[0], kappa, M0[t], Mb[t], S32[t]);
-    }
-    else
-    {
-      // one kernel per group: the lower half keeps even point tiles, the
-      // upper half odd ones; state q of a lane is its tile 2 q + g
-      const float tot = halfwave_pair_sum (part[0], part[0]) * sc2;
-
-      if (t & 1)
+      if (rg == P::NRG - 1)
       {
-        const float mine = g ? tot : tot_prev;
-
-        lse_push<KERNEL, OFFSET> (mine, cur.cf[0], kappa, M0[t / 2], Mb[t / 2], S32[t / 2]);
-      }
-      else
-      {
-        tot_prev = tot;
+#pragma unroll
+        for (int j = 0; j < P::NLOCAL; ++j)
+          lse_push<KERNEL, OFFSET> (SCALED ? part[t][j] * it2[t] : part[t][j], cf[j], kappa, M0[t], Mb[t], S32[t]);
       }
     }
+
+    if (DP >= 16)
+      __builtin_amdgcn_sched_barrier (0);
   }
 }
 
-// Tiling chosen by measurement on MI355X: up to DP = 16 a wave keeps more
-// point tiles and loads each kernel group just before its MFMA chains (the
-// occupancy of the smaller register set hides the loads).  At DP = 32 the
-// next kernel is prefetched into a second register set.  At DP = 64 one
-// kernel's factors (16 KiB) feed all four waves of a block: they are staged
-// once per block in LDS, double-buffered, the next kernel's global loads in
-// flight while the current one is computed (1.5x faster than the register
-// prefetch at d = 64; at d = 32 the barrier per kernel costs more than the
-// shared loads save).
+// Tiling chosen by measurement on MI355X: up to DP = 16 a wave loads each
+// row tile just before its MFMA chains (two to four waves per SIMD hide the
+// loads); at DP = 16 six point tiles are the most that leave two waves (n =
+// 20000, m = 200000: 4.83 ms, 5.13 with four, 5.44 with eight).  At DP = 32 the
+// next row tile is prefetched into a second register set.  At DP = 64 a
+// group's factors (32 KiB) feed all eight waves of a block: they are staged
+// once per block in LDS, double-buffered, the next group's global loads in
+// flight while the current one is computed.
 constexpr int
 tiles_per_wave (int DP)
 {
-  return (DP == 64) ? 2 : ((DP == 16) ? 8 : 4);
+  return (DP == 64) ? 2 : ((DP == 16) ? 6 : 4);
 }
 
 constexpr bool
@@ -714,16 +703,17 @@ waves_per_block (int DP)
   return (DP == 64) ? 8 : 4;
 }
 
-// LDS stage of one kernel (DP = 64): A hi rows then lo rows, each padded to
-// DP + 8 halves (16 B) so that the 32 rows read by a fragment load spread
-// over the banks; then c (DP floats) and the coefficients.
+// LDS stage of one group (DP = 64): per kernel A hi rows then lo rows, each
+// padded to DP + 8 halves (16 B) so that the 16 rows read by a fragment load
+// spread over the banks; then c (DP floats per kernel) and the coefficients.
 template <int DP>
 struct Stage
 {
   static constexpr int RS  = DP + 8;                  // row stride, halves
-  static constexpr int ASZ = 2 * DP * RS;             // halves per stage
+  static constexpr int KPT = Plan<DP>::KPT;
+  static constexpr int ASZ = KPT * 2 * DP * RS;       // halves per stage
   static constexpr int NT  = 64 * waves_per_block (DP);   // threads per block
-  static constexpr int CPT = 2 * DP * DP / 8 / NT;        // 16 B chunks per thread
+  static constexpr int CPT = KPT * 2 * DP * DP / 8 / NT;  // 16 B chunks per thread
 };
 
 typedef unsigned int u32x4 __attribute__ ((ext_vector_type (4)));
@@ -742,15 +732,16 @@ __device__ inline void
 stage_load (StageFetch<DP> &s, const _Float16 *__restrict__ A, const float *__restrict__ cv,
             const float4 *__restrict__ coef, int tg, int tid)
 {
-  const u32x4 *src = (const u32x4 *) (A + (size_t) tg * 2 * DP * DP);
+  constexpr int KPT = Plan<DP>::KPT;
+  const u32x4 *src  = (const u32x4 *) (A + (size_t) tg * KPT * 2 * DP * DP);
 
 #pragma unroll
   for (int q = 0; q < Stage<DP>::CPT; ++q)
     s.a[q] = src[tid + q * Stage<DP>::NT];
 
   // every thread loads (in bounds) so the stage stays in registers
-  s.c = ((const f32x4 *) (cv + (size_t) tg * DP))[tid % (DP / 4)];
-  s.f = ((const f32x4 *) coef)[tg];
+  s.c = ((const f32x4 *) (cv + (size_t) tg * KPT * DP))[tid % (KPT * DP / 4)];
+  s.f = ((const f32x4 *) coef)[tg * KPT + tid % KPT];
 }
 
 template <int DP>
@@ -767,188 +758,215 @@ stage_store (const StageFetch<DP> &s, _Float16 *sA, float *sC, float4 *sF, int t
     *(u32x4 *) (sA + (e / CPR) * Stage<DP>::RS + (e % CPR) * 8) = s.a[q];
   }
 
-  if (tid < DP / 4)
+  if (tid < Plan<DP>::KPT * DP / 4)
     ((f32x4 *) sC)[tid] = s.c;
 
-  if (tid == 0)
-    *(f32x4 *) sF = s.f;
+  if (tid < Plan<DP>::KPT)
+    ((f32x4 *) sF)[tid] = s.f;
 }
 
-// the fragments of a staged kernel, as load_group reads them from global memory
-template <int DP>
+// group_step of a staged group: both point tiles of a row tile together, their
+// A fragments read from LDS K block by K block, the norms one row tile behind
+// the MFMA chains.
+template <int DP, int KERNEL, int NPT, bool OFFSET, bool SCALED>
 __device__ inline void
-load_group_lds (GroupData<DP> &G, const _Float16 *sA, const float *sC, const float4 *sF, int lane)
+group_step_lds (const _Float16 *sA, const float *sC, const float4 *sF, const PointFrag<DP> (&B)[NPT],
+                const float (&tscale)[NPT], const float (&it2)[NPT], const float (&M0)[NPT], float (&Mb)[NPT],
+                float (&S32)[NPT], float kappa, int lane)
 {
-  using P            = Plan<DP>;
-  constexpr int RS   = Stage<DP>::RS;
-  const unsigned g   = lane >> 5;
-  const unsigned R   = lane & 31;
+  using P          = Plan<DP>;
+  constexpr int RS = Stage<DP>::RS;
+  const unsigned g = lane >> 5;
+  unsigned kl, dim;
+
+  tile_row<DP> (lane & 31, kl, dim);
+
+  const _Float16 *a = sA + (kl * 2 * DP + dim) * RS + g * 8;
+  const float *c    = sC + g * DP;
+  const float4 cf   = sF[g];
+  floatx16 acc[2][NPT];
+  float part[NPT];
 
 #pragma unroll
-  for (int rt = 0; rt < P::NRT; ++rt)
+  for (int rg = 0; rg <= P::NRG; ++rg)
   {
-    const unsigned row = (DP == 64) ? rt * 32 + R : R;
+    if (rg < P::NRG)
+    {
+      floatx16 c0;
 
 #pragma unroll
-    for (int kb = 0; kb < P::NKB; ++kb)
-    {
-      G.Ah[rt][kb] = *(const half8 *) (sA + row * RS + kb * 16 + g * 8);
-      G.Al[rt][kb] = *(const half8 *) (sA + (DP + row) * RS + kb * 16 + g * 8);
-    }
+      for (int j = 0; j < 4; ++j)
+      {
+        const float4 c4 = *(const float4 *) (c + rg * 16 + 4 * j);
+
+        c0[4 * j + 0] = c4.x;
+        c0[4 * j + 1] = c4.y;
+        c0[4 * j + 2] = c4.z;
+        c0[4 * j + 3] = c4.w;
+      }
 
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-    {
-      const unsigned Rr = 8 * j + 4 * g;
-      const float4 c4   = *(const float4 *) (sC + ((DP == 64) ? rt * 32 + Rr : Rr));
+      for (int t = 0; t < NPT; ++t)
+      {
+        floatx16 z = c0;
 
-      G.cinit[rt][4 * j + 0] = c4.x;
-      G.cinit[rt][4 * j + 1] = c4.y;
-      G.cinit[rt][4 * j + 2] = c4.z;
-      G.cinit[rt][4 * j + 3] = c4.w;
+        if (SCALED)
+        {
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            z[r] *= tscale[t];
+        }
+
+        acc[rg & 1][t] = z;
+      }
+
+#pragma unroll
+      for (int kb = 0; kb <= rg; ++kb)
+      {
+        const half8 h = *(const half8 *) (a + rg * 16 * RS + kb * 16);
+        const half8 l = *(const half8 *) (a + (DP + rg * 16) * RS + kb * 16);
+
+#pragma unroll
+        for (int t = 0; t < NPT; ++t)
+          acc[rg & 1][t] = mixed_mfma (h, B[t].h[kb], acc[rg & 1][t]);
+
+#pragma unroll
+        for (int t = 0; t < NPT; ++t)
+          acc[rg & 1][t] = mixed_mfma (h, B[t].l[kb], acc[rg & 1][t]);
+
+#pragma unroll
+        for (int t = 0; t < NPT; ++t)
+          acc[rg & 1][t] = mixed_mfma (l, B[t].h[kb], acc[rg & 1][t]);
+      }
     }
+
+    if (rg > 0)
+    {
+#pragma unroll
+      for (int t = 0; t < NPT; ++t)
+      {
+        const floatx16 &z = acc[(rg - 1) & 1][t];
+        float p           = z[0] * z[0];
+
+#pragma unroll
+        for (int r = 1; r < 16; ++r)
+          p = fmaf (z[r], z[r], p);
+
+        part[t] = (rg == 1) ? p : part[t] + p;
+
+        if (rg == P::NRG)
+          lse_push<KERNEL, OFFSET> (SCALED ? part[t] * it2[t] : part[t], cf, kappa, M0[t], Mb[t], S32[t]);
+      }
+    }
+
+    __builtin_amdgcn_sched_barrier (0);
   }
-
-#pragma unroll
-  for (int q = 0; q < 4; ++q)
-    G.cf[q] = *sF;
 }
 
-template <int DP, int KERNEL, int NPT, bool OFFSET, bool SCALED, int NST>
+template <int DP, int KERNEL, int NPT, bool OFFSET, bool SCALED>
 __device__ inline void
 group_loop (int g0, int g1, const _Float16 *__restrict__ A, const float *__restrict__ cv,
-            const float4 *__restrict__ coef, const half8 (&Bh)[NPT][Plan<DP>::NKB],
-            const half8 (&Bl)[NPT][Plan<DP>::NKB], const float (&tscale)[NPT], const float (&it2)[NPT],
-            const float (&M0)[NST], float (&Mb)[NST], double (&S64)[NST], float kappa, int lane,
+            const float4 *__restrict__ coef, const PointFrag<DP> (&B)[NPT], const float (&tscale)[NPT], const float (&it2)[NPT],
+            const float (&M0)[NPT], float (&Mb)[NPT], double (&S64)[NPT], float kappa, int lane,
             _Float16 *sA, float *sC, float4 *sF)
 {
-  const int g = lane >> 5;
-  float S32[NST];
+  using P = Plan<DP>;
+  float S32[NPT];
+  constexpr int NG = (DP == 32) ? 2 : 1;
+  RowData<DP> G[NG];
+  float4 cf[P::NLOCAL];
 
 #pragma unroll
-  for (int q = 0; q < NST; ++q)
+  for (int q = 0; q < NPT; ++q)
     S32[q] = 0.0f;
 
-  if constexpr (DP <= 16)
-  {
-    for (int tg = g0; tg < g1; ++tg)
-    {
-      GroupData<DP> gd;
-
-      load_group<DP> (gd, A, cv, coef, tg, lane);
-      group_step<DP, KERNEL, NPT, OFFSET, SCALED, NST> (gd, Bh, Bl, tscale, it2, M0, Mb, S32, kappa, g);
-
-      // fold the FP32 partial sums into FP64 every 16 groups
-      if (((tg + 1 - g0) & 15) == 0)
-      {
-#pragma unroll
-        for (int q = 0; q < NST; ++q)
-        {
-          S64[q] += (double) S32[q];
-          S32[q] = 0.0f;
-        }
-      }
-    }
-
-#pragma unroll
-    for (int q = 0; q < NST; ++q)
-      S64[q] += (double) S32[q];
-  }
-  else if constexpr (!lds_groups (DP))
-  {
-    // two register sets alternate roles: while one group is computed the
-    // next one is loaded into the other set (no register copies)
-    GroupData<DP> ga, gb;
-    int tg = g0;
-
-    if (tg < g1)
-      load_group<DP> (ga, A, cv, coef, tg, lane);
-
-    while (tg < g1)
-    {
-      if (tg + 1 < g1)
-        load_group<DP> (gb, A, cv, coef, tg + 1, lane);
-
-      group_step<DP, KERNEL, NPT, OFFSET, SCALED, NST> (ga, Bh, Bl, tscale, it2, M0, Mb, S32, kappa, g);
-      ++tg;
-
-      if (tg >= g1)
-        break;
-
-      if (tg + 1 < g1)
-        load_group<DP> (ga, A, cv, coef, tg + 1, lane);
-
-      group_step<DP, KERNEL, NPT, OFFSET, SCALED, NST> (gb, Bh, Bl, tscale, it2, M0, Mb, S32, kappa, g);
-      ++tg;
-
-      // fold the FP32 partial sums into FP64 every 16 groups
-      if (((tg - g0) & 15) == 0)
-      {
-#pragma unroll
-        for (int q = 0; q < NST; ++q)
-        {
-          S64[q] += (double) S32[q];
-          S32[q] = 0.0f;
-        }
-      }
-    }
-
-#pragma unroll
-    for (int q = 0; q < NST; ++q)
-      S64[q] += (double) S32[q];
-  }
-  else
-  {
-  // staged groups: g0 and g1 are block-uniform, so every wave of the block
-  // runs the same iterations and meets the same barriers.  Stage st is read
-  // in iteration tg while the other one is written; the barrier at the end of
-  // each iteration orders those reads before the next overwrite.
-  const int tid = threadIdx.x;
-  StageFetch<DP> nx;
-
-  if (g0 < g1)
-  {
-    stage_load<DP> (nx, A, cv, coef, g0, tid);
-    stage_store<DP> (nx, sA, sC, sF, tid);
-  }
-
-  __syncthreads ();
-
-  for (int tg = g0; tg < g1; ++tg)
-  {
-    const int st = (tg - g0) & 1;
-
-    if (tg + 1 < g1)
-      stage_load<DP> (nx, A, cv, coef, tg + 1, tid);
-
-    {
-      GroupData<DP> gd;
-
-      load_group_lds<DP> (gd, sA + st * Stage<DP>::ASZ, sC + st * DP, sF + st, lane);
-      group_step<DP, KERNEL, NPT, OFFSET, SCALED, NST> (gd, Bh, Bl, tscale, it2, M0, Mb, S32, kappa, g);
-    }
-
-    if (tg + 1 < g1)
-      stage_store<DP> (nx, sA + (st ^ 1) * Stage<DP>::ASZ, sC + (st ^ 1) * DP, sF + (st ^ 1), tid);
-
-    __syncthreads ();
-
-    // fold the FP32 partial sums into FP64 every 16 groups
-    if (((tg + 1 - g0) & 15) == 0)
+  // fold the FP32 partial sums into FP64 every 16 groups (8 at DP = 16): after
+  // 16 terms of a lane from DP = 16 on, 32 at DP = 8, 64 at DP = 4
+  auto fold = [&] (int done) {
+    if ((done & ((DP == 16) ? 7 : 15)) == 0)
     {
 #pragma unroll
-      for (int q = 0; q < NST; ++q)
+      for (int q = 0; q < NPT; ++q)
       {
         S64[q] += (double) S32[q];
         S32[q] = 0.0f;
       }
     }
+  };
+
+  if constexpr (DP <= 16)
+  {
+    for (int tg = g0; tg < g1; ++tg)
+    {
+      load_coef<DP> (cf, coef, tg, lane);
+      group_step<DP, KERNEL, NPT, OFFSET, SCALED> (G, cf, B, tscale, it2, M0, Mb, S32, kappa,
+                                                   [&] (RowData<DP> (&n)[NG], int rg) {
+                                                     load_rows<DP> (n[0], A, cv, tg, rg, lane);
+                                                   });
+      fold (tg + 1 - g0);
+    }
+  }
+  else if constexpr (!lds_groups (DP))
+  {
+    if (g0 < g1)
+      load_rows<DP> (G[0], A, cv, g0, 0, lane);
+
+    for (int tg = g0; tg < g1; ++tg)
+    {
+      const int tn = min (tg + 1, g1 - 1);   // the last group loads its first rows again
+
+      load_coef<DP> (cf, coef, tg, lane);
+      group_step<DP, KERNEL, NPT, OFFSET, SCALED> (G, cf, B, tscale, it2, M0, Mb, S32, kappa,
+                                                   [&] (RowData<DP> (&n)[NG], int rg) {
+                                                     if (rg + 1 < P::NRG)
+                                                       load_rows<DP> (n[(rg + 1) % NG], A, cv, tg, rg + 1, lane);
+                                                     else
+                                                       load_rows<DP> (n[(rg + 1) % NG], A, cv, tn, 0, lane);
+                                                   });
+      fold (tg + 1 - g0);
+    }
+  }
+  else
+  {
+    // staged groups: g0 and g1 are block-uniform, so every wave of the block
+    // runs the same iterations and meets the same barriers.  Stage st is read
+    // in iteration tg while the other one is written; the barrier at the end
+    // of each iteration orders those reads before the next overwrite.
+    const int tid = threadIdx.x;
+    StageFetch<DP> nx;
+
+    if (g0 < g1)
+    {
+      stage_load<DP> (nx, A, cv, coef, g0, tid);
+      stage_store<DP> (nx, sA, sC, sF, tid);
+    }
+
+    __syncthreads ();
+
+    for (int tg = g0; tg < g1; ++tg)
+    {
+      const int st        = (tg - g0) & 1;
+      const _Float16 *cA  = sA + st * Stage<DP>::ASZ;
+      const float *cC     = sC + st * P::KPT * DP;
+
+      if (tg + 1 < g1)
+        stage_load<DP> (nx, A, cv, coef, tg + 1, tid);
+
+      group_step_lds<DP, KERNEL, NPT, OFFSET, SCALED> (cA, cC, sF + st * P::KPT, B, tscale, it2, M0, Mb, S32,
+                                                       kappa, lane);
+
+      if (tg + 1 < g1)
+        stage_store<DP> (nx, sA + (st ^ 1) * Stage<DP>::ASZ, sC + (st ^ 1) * P::KPT * DP, sF + (st ^ 1) * P::KPT,
+                         tid);
+
+      __syncthreads ();
+      fold (tg + 1 - g0);
+    }
   }
 
 #pragma unroll
-  for (int q = 0; q < NST; ++q)
+  for (int q = 0; q < NPT; ++q)
     S64[q] += (double) S32[q];
-  }
 }
 
 // The evaluation of one block: block (bx, by) takes the point tiles of
@@ -958,7 +976,6 @@ __device__ inline void
 eval_mixed_block (const MixedArgs &a, int bx, int by)
 {
   using P        = Plan<DP>;
-  constexpr int NST = (DP >= 32) ? NPT / 2 : NPT;   // LSE states per lane
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int g    = lane >> 5;
@@ -979,10 +996,10 @@ eval_mixed_block (const MixedArgs &a, int bx, int by)
   const int g1      = min (ngroups, g0 + chunk);
 
   // second pass: only waves holding a flagged point do any work
-  float M0[NST];
+  float M0[NPT];
 
 #pragma unroll
-  for (int q = 0; q < NST; ++q)
+  for (int q = 0; q < NPT; ++q)
     M0[q] = 0.0f;
 
   if (OFFSET)
@@ -1003,17 +1020,16 @@ eval_mixed_block (const MixedArgs &a, int bx, int by)
       return;
 
 #pragma unroll
-    for (int q = 0; q < NST; ++q)
+    for (int q = 0; q < NPT; ++q)
     {
-      const int t = (DP >= 32) ? 2 * q + g : q;
-      const int p = min ((tile0 + t) * 32 + R, a.m - 1);
+      const int p = min ((tile0 + q) * 32 + R, a.m - 1);
 
       M0[q] = a.M0[p];
     }
   }
 
   // B fragments (points) and per-point scales
-  half8 Bh[NPT][P::NKB], Bl[NPT][P::NKB];
+  PointFrag<DP> B[NPT];
   float tscale[NPT], it2[NPT];
   bool scaled = false;
 
@@ -1024,12 +1040,7 @@ eval_mixed_block (const MixedArgs &a, int bx, int by)
 
     p = (p < a.m) ? p : a.m - 1;
 
-#pragma unroll
-    for (int kb = 0; kb < P::NKB; ++kb)
-    {
-      Bh[t][kb] = load_b_frag<DP> (Yh, Yl, p, kb, 0, lane);
-      Bl[t][kb] = load_b_frag<DP> (Yh, Yl, p, kb, 1, lane);
-    }
+    load_points<DP> (B[t], Yh, Yl, p, lane);
 
     const float2 tv = tpv[p];
 
@@ -1038,47 +1049,30 @@ eval_mixed_block (const MixedArgs &a, int bx, int by)
     scaled    = scaled || (tv.x != 1.0f);
   }
 
-  float Mb[NST];
-  double S64[NST];
+  float Mb[NPT];
+  double S64[NPT];
 
 #pragma unroll
-  for (int q = 0; q < NST; ++q)
+  for (int q = 0; q < NPT; ++q)
   {
     Mb[q]  = -INFINITY;
     S64[q] = 0.0;
   }
 
-  // LDS stages of the factors (DP >= 32), two per block
+  // LDS stages of the factors (DP = 64), two per block
   __shared__ __attribute__ ((aligned (16))) _Float16 sA[lds_groups (DP) ? 2 * Stage<DP>::ASZ : 8];
-  __shared__ __attribute__ ((aligned (16))) float sC[lds_groups (DP) ? 2 * DP : 4];
-  __shared__ float4 sF[2];
+  __shared__ __attribute__ ((aligned (16))) float sC[lds_groups (DP) ? 2 * P::KPT * DP : 4];
+  __shared__ float4 sF[2 * P::KPT];
 
   // the scaled/unscaled choice is block-wide where the loop has barriers
   const bool any_scaled = lds_groups (DP) ? (bool) __syncthreads_or (scaled) : (bool) __any (scaled);
 
   if (any_scaled)
-    group_loop<DP, KERNEL, NPT, OFFSET, true, NST> (g0, g1, A, cv, coef, Bh, Bl, tscale, it2, M0, Mb, S64, kappa,
-                                                    lane, sA, sC, sF);
+    group_loop<DP, KERNEL, NPT, OFFSET, true> (g0, g1, A, cv, coef, B, tscale, it2, M0, Mb, S64, kappa, lane, sA,
+                                               sC, sF);
   else
-    group_loop<DP, KERNEL, NPT, OFFSET, false, NST> (g0, g1, A, cv, coef, Bh, Bl, tscale, it2, M0, Mb, S64, kappa,
-                                                     lane, sA, sC, sF);
-
-  if (DP >= 32)
-  {
-#pragma unroll
-    for (int q = 0; q < NST; ++q)
-    {
-      const int p = (tile0 + 2 * q + g) * 32 + R;
-
-      if (p < a.m)
-      {
-        a.partM[(size_t) by * a.m + p] = Mb[q];
-        a.partS[(size_t) by * a.m + p] = S64[q];
-      }
-    }
-
-    return;
-  }
+    group_loop<DP, KERNEL, NPT, OFFSET, false> (g0, g1, A, cv, coef, B, tscale, it2, M0, Mb, S64, kappa, lane,
+                                                sA, sC, sF);
 
   // the two half-waves hold the same points (disjoint kernel slots) and the
   // same reference: add the sums, take the larger maximum
@@ -1419,7 +1413,7 @@ mixed_build (const double *X, int n, int d, int D, int DP, const double *Wp, con
   // the sample's largest |y'| maps to about 2^11: eval points up to 8x
   // farther out need no per-point rescaling
   const double ysc = (ymax > 0.0) ? ldexp (1.0, 11 - ilogb (ymax) - 1) : 1.0;
-  const int kpt    = (DP >= 32) ? 1 : 32 / DP;
+  const int kpt    = mixed_group (DP);
   const int n_pad  = ((n + kpt - 1) / kpt) * kpt;
 
   *ysc_out = ysc;

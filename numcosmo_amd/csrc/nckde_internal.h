@@ -252,6 +252,12 @@ enum MixedMerge
   MERGE_CHECK   = 3,  // terms against the pilot reference: results; points whose largest term is too far
                       // above it (or whose sum is not finite) flagged, with their maxima
 };
+// kernels per group of the mixed eval (the factors are padded to whole groups)
+constexpr int
+mixed_group (int DP)
+{
+  return (DP == 4) ? 8 : (DP <= 16) ? 4 : 2;
+}
 int mixed_points_per_block (int DP);
 hipError_t launch_mixed_points (const MixedArgs &a, hipStream_t s);
 hipError_t launch_eval_mixed (const MixedArgs &a, hipStream_t s);

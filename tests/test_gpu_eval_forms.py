@@ -97,3 +97,18 @@ def test_interpolation_matrix(oracle, nu, d, n):
     sd, od = _pair(oracle, 1, nu, d, X)
     got, ref = sd.compute_IM(), od.compute_IM()
     assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1e-300)) < 1e-11
+
+
+@pytest.mark.parametrize("nu", [0.0, 3.0])
+@pytest.mark.parametrize("d,n", [(3, 129), (8, 130), (9, 131), (12, 161), (16, 162), (16, 163), (17, 321), (32, 322),
+                                 (33, 323), (48, 324), (64, 325), (64, 1027)])
+@pytest.mark.parametrize("m", [1, 33, 800])
+def test_mixed_groups(oracle, nu, d, n, m):
+    """Mixed evals with kernel counts that leave part of a group, and point
+    counts around the 32-point tiles: 1e-6 relative, the bar of the mixed path."""
+    g = np.random.default_rng(d * n + m)
+    X = g.normal(size=(n, d))
+    sd, od = _pair(oracle, 1, nu, d, X)
+    P = np.concatenate([g.normal(size=(m, d)), X[:1], 40.0 * g.normal(size=(1, d))])
+    got, ref = sd.eval_m2lnp_batch(P, 1), od.eval_m2lnp_batch(P)
+    assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-6
