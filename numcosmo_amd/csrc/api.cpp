@@ -1466,7 +1466,13 @@ fp64_nsplit (const nckde *h, size_t m, int prec)
 
   const int nblk = (int) ((m + 255) / 256);
   int nsplit     = (16384 + nblk - 1) / nblk;
-  const int maxs = (int) ((h->n_k + 31) / 32);
+  int maxs       = (int) ((h->n_k + 31) / 32);
+
+  // up to 2048 points: a split's kernels run one after the other, so splits go
+  // down to 4 kernels while the grid stays below 2048 blocks (n = 1000, d = 4:
+  // one point 41 -> 35 us; at 10000 points the larger merge costs more)
+  if (m <= 2048)
+    maxs = std::max (maxs, std::min ((int) ((h->n_k + 3) / 4), 2048 / nblk));
 
   return std::max (1, std::min (nsplit, maxs));
 }
@@ -1614,6 +1620,18 @@ template <class Run>
 static int eval_graph (nckde *h, const double *dX, size_t m, double *dout, int precision, int linear, hipStream_t s,
                        const Run &run);
 
+// Mixed evals that the FP64 form finishes sooner: its two launches against the
+// mixed form's five, and splits of few kernels against its groups (measured
+// per call at n = 600 / 3000 / 20000: d = 6, m = 64: 9 / 12 / 22 us against 16 /
+// 19 / 42; d = 16, m = 256: 13 / 28 / 89 against 23 / 30 / 86; d = 40, m = 256:
+// 25 / 64 / 314 against 74 / - / 378; d = 3, m = 128: 9 / 16 / 35 against 17 / 17 /
+// 29).  The factors are built all the same.
+static bool
+mixed_small (const nckde *h, size_t m)
+{
+  return m <= 64 || (h->d > 4 && m <= 128) || (h->d >= 13 && m <= 256) || m * h->n_k <= 750000;
+}
+
 static int
 eval_device (nckde *h, const double *dX, size_t m, double *dout, int precision, int linear, hipStream_t s)
 {
@@ -1634,7 +1652,7 @@ eval_device (nckde *h, const double *dX, size_t m, double *dout, int precision, 
   {
     TRY (ensure_mixed (h));
 
-    if (h->mixed_fallback)
+    if (h->mixed_fallback || mixed_small (h, m))
       precision = NCKDE_PREC_FP64;
   }
   else if (precision == NCKDE_PREC_FP32)
@@ -3149,7 +3167,7 @@ nckde_eval_m2lnp_device_noalloc (nckde *h, const double *dX, size_t m, double *d
       return NCKDE_ESTATE;
     }
 
-    if (h->mixed_fallback)
+    if (h->mixed_fallback || mixed_small (h, m))
       precision = NCKDE_PREC_FP64;
   }
 
@@ -3270,7 +3288,7 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
     if (fuse)
     {
       TRY (ensure_mixed (h));
-      fuse = !h->mixed_fallback && h->pilot_n == 0;
+      fuse = !h->mixed_fallback && h->pilot_n == 0 && !mixed_small (h, m[i]);
     }
 
     if (!fuse)
