@@ -250,17 +250,10 @@ launch_transpose (const double *in, int rows, int cols, double *out, hipStream_t
 // over BM x BM tiles of the upper triangle.  256 threads = 4 waves in a
 // 2 x 2 layout, each wave a BM/2 x BM/2 block of 16 x 16 MFMA tiles; K
 // staged through LDS in slices of 16, the next slice's global loads in
-// flight during the current slice's MFMAs.  BM = 128 serves large products
-// (at least 1024 tiles for the Gram matrix, 16384 for the Cholesky update)
-// and BM = 64 the smaller ones: 4x more blocks, and for the Cholesky update
-// (K = 64) a 4x shorter MFMA chain per block, which suits the shrinking
-// trailing matrix.
-//   mode 0: M = AT AT^T (AT is n x K row-major): the Gram matrix A^T A of
-//           the NNLS normal equations (cblas_dsyrk, ncm_matrix.c:1547-1575);
-//           both triangles are written.
-//   mode 1: trailing update of the Cholesky's super-panels (k_potrf.hip),
-//           S[a][b] -= sum_r S[kb+r][a] S[kb+r][b] over the rows
-//           kb..kb+K-1, for off <= a <= b (upper triangle only).
+// flight during the current slice's MFMAs.  k_gram forms the Gram matrix of
+// the normal equations, k_syrk_mfma the trailing update of the Cholesky's
+// super-panels (k_potrf.hip): S[a][b] -= sum_r S[kb+r][a] S[kb+r][b] over the
+// rows kb..kb+K-1, for off <= a <= b (upper triangle only).
 // Tiles are numbered along the rows of the upper triangle; the grid is
 // padded to a multiple of 8 and block b takes tile (b % 8) * (grid / 8) +
 // b / 8, so that each XCD (blocks are dealt round-robin over the 8 XCDs)
@@ -268,65 +261,40 @@ launch_transpose (const double *in, int rows, int cols, double *out, hipStream_t
 // --------------------------------------------------------------------------
 typedef double f64x4 __attribute__ ((ext_vector_type (4)));
 
-constexpr int SY_BM = 128;   // tile of the Gram matrix (MODE 0)
 constexpr int SY_BK = 16;
 
 // BM: square tile of one block (128 or 64); every thread stages
 // VPT = 16 BM / 256 values of each operand per K slice, 16 threads per K row
-template <int MODE, int BM>
+template <int BM>
 __device__ inline void
 syrk_load (const double *__restrict__ P, int n, int K, int ld, int kb, int r0, int k0, double (&v)[BM / 16])
 {
   constexpr int VPT = BM / 16;
   const int tid     = threadIdx.x;
 
-  if (MODE == 0)
-  {
-    // 256 / BM threads per row, VPT consecutive K entries each
-    const int a  = r0 + tid / (256 / BM);
-    const int kq = k0 + (tid % (256 / BM)) * VPT;
+  const int kq = k0 + tid / 16;
+  const int a  = r0 + (tid % 16) * VPT;
 
 #pragma unroll
-    for (int q = 0; q < VPT; ++q)
-      v[q] = (a < n && kq + q < K) ? P[(size_t) a * ld + kq + q] : 0.0;
-  }
-  else
-  {
-    const int kq = k0 + tid / 16;
-    const int a  = r0 + (tid % 16) * VPT;
-
-#pragma unroll
-    for (int q = 0; q < VPT; ++q)
-      v[q] = (a + q < n && kq < K) ? P[(size_t) (kb + kq) * ld + a + q] : 0.0;
-  }
+  for (int q = 0; q < VPT; ++q)
+    v[q] = (a + q < n && kq < K) ? P[(size_t) (kb + kq) * ld + a + q] : 0.0;
 }
 
-template <int MODE, int BM>
+template <int BM>
 __device__ inline void
 syrk_store (double (*T)[BM + 4], const double (&v)[BM / 16])
 {
   constexpr int VPT = BM / 16;
   const int tid     = threadIdx.x;
 
-  if (MODE == 0)
-  {
-    const int rr = tid / (256 / BM), kk = (tid % (256 / BM)) * VPT;
+  const int kk = tid / 16, rr = (tid % 16) * VPT;
 
 #pragma unroll
-    for (int q = 0; q < VPT; ++q)
-      T[kk + q][rr] = v[q];
-  }
-  else
-  {
-    const int kk = tid / 16, rr = (tid % 16) * VPT;
-
-#pragma unroll
-    for (int q = 0; q < VPT; ++q)
-      T[kk][rr + q] = v[q];
-  }
+  for (int q = 0; q < VPT; ++q)
+    T[kk][rr + q] = v[q];
 }
 
-template <int MODE, int BM>
+template <int BM>
 __global__ void __launch_bounds__ (256)
 k_syrk_mfma (const double *__restrict__ P, int n, int K, int ld, int off, int kb, double *__restrict__ M,
              int ntiles)
@@ -369,20 +337,20 @@ k_syrk_mfma (const double *__restrict__ P, int n, int K, int ld, int off, int kb
 
   double va[BM / 16], vb[BM / 16];
 
-  syrk_load<MODE, BM> (P, n, K, ld, kb, r0, 0, va);
-  syrk_load<MODE, BM> (P, n, K, ld, kb, c0, 0, vb);
+  syrk_load<BM> (P, n, K, ld, kb, r0, 0, va);
+  syrk_load<BM> (P, n, K, ld, kb, c0, 0, vb);
 
   for (int k0 = 0; k0 < K; k0 += SY_BK)
   {
     __syncthreads ();
-    syrk_store<MODE, BM> (As, va);
-    syrk_store<MODE, BM> (Bs, vb);
+    syrk_store<BM> (As, va);
+    syrk_store<BM> (Bs, vb);
     __syncthreads ();
 
     if (k0 + SY_BK < K)
     {
-      syrk_load<MODE, BM> (P, n, K, ld, kb, r0, k0 + SY_BK, va);
-      syrk_load<MODE, BM> (P, n, K, ld, kb, c0, k0 + SY_BK, vb);
+      syrk_load<BM> (P, n, K, ld, kb, r0, k0 + SY_BK, va);
+      syrk_load<BM> (P, n, K, ld, kb, c0, k0 + SY_BK, vb);
     }
 
 #pragma unroll
@@ -407,61 +375,177 @@ k_syrk_mfma (const double *__restrict__ P, int n, int K, int ld, int off, int kb
   }
 
   // D[i][j] of a 16 x 16 tile: register r of a lane holds i = lane / 16 + 4 r, j = lane % 16
-  if (MODE == 0)
+  // read-modify-write of the tile, one 16-column block at a time with all
+  // loads of a lane in flight (out-of-range entries read element 0)
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
   {
+    const int b = c0 + wc + j * 16 + li;
+    double old[NI][4];
+
 #pragma unroll
     for (int i = 0; i < NI; ++i)
 #pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-          const int a = r0 + wr + i * 16 + lk + 4 * r;
-          const int b = c0 + wc + j * 16 + li;
+      for (int r = 0; r < 4; ++r)
+      {
+        const int a  = r0 + wr + i * 16 + lk + 4 * r;
+        const bool v = (a < n && b < n && a <= b);
 
-          if (a < n && b < n && a <= b)
-          {
-            M[(size_t) a * n + b] = acc[i][j][r];
-            M[(size_t) b * n + a] = acc[i][j][r];
-          }
-        }
-  }
-  else
-  {
-    // read-modify-write of the tile, one 16-column block at a time with all
-    // loads of a lane in flight (out-of-range entries read element 0)
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-    {
-      const int b = c0 + wc + j * 16 + li;
-      double old[NI][4];
+        old[i][r] = M[v ? (size_t) a * ld + b : 0];
+      }
 
 #pragma unroll
-      for (int i = 0; i < NI; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-          const int a  = r0 + wr + i * 16 + lk + 4 * r;
-          const bool v = (a < n && b < n && a <= b);
+      for (int r = 0; r < 4; ++r)
+      {
+        const int a = r0 + wr + i * 16 + lk + 4 * r;
 
-          old[i][r] = M[v ? (size_t) a * ld + b : 0];
-        }
-
-#pragma unroll
-      for (int i = 0; i < NI; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-        {
-          const int a = r0 + wr + i * 16 + lk + 4 * r;
-
-          if (a < n && b < n && a <= b)
-            M[(size_t) a * ld + b] = old[i][r] - acc[i][j][r];
-        }
-    }
+        if (a < n && b < n && a <= b)
+          M[(size_t) a * ld + b] = old[i][r] - acc[i][j][r];
+      }
   }
 }
 
-template <int MODE, int BM = SY_BM>
+// Gram matrix M = AT AT^T (AT is n x K row-major): A^T A of the NNLS normal
+// equations (cblas_dsyrk, ncm_matrix.c:1547-1575), both triangles written.
+// Slices of 16 columns in two LDS buffers, one barrier per slice, the next
+// slice's loads in flight under the MFMAs; 16 threads read a row's 128 bytes,
+// which stays coalesced for odd K.  n = 10000: 18.4 -> 17.4 ms, n = 2503: 0.46
+// -> 0.39 ms against the transposing stage of k_syrk_mfma (57 TFLOP/s of a
+// library GEMM's 72).
+template <int BM>
+__global__ void __launch_bounds__ (256)
+k_gram (const double *__restrict__ P, int n, int K, double *__restrict__ M, int ntiles)
+{
+  static_assert (BM == 128 || BM == 64, "128- or 64-wide tiles");
+  constexpr int WM = BM / 2, NI = WM / 16;      // tile of one wave, its 16 x 16 MFMA blocks per dimension
+  constexpr int BK = SY_BK, LD = BK + 2;        // row stride in LDS: 16 rows x 4 columns hit every bank once per cycle
+  constexpr int RPT = 256 / BK, VPT = BM / RPT; // staged rows per pass, entries per thread
+  __shared__ double As[2][BM][LD];
+  __shared__ double Bs[2][BM][LD];
+  const int per = gridDim.x / 8;
+  int t         = (blockIdx.x % 8) * per + blockIdx.x / 8;
+
+  if (t >= ntiles)
+    return;
+
+  const int nt = (n + BM - 1) / BM;
+  int ti       = 0;
+
+  while (t >= nt - ti)
+  {
+    t -= nt - ti;
+    ++ti;
+  }
+
+  const int r0   = ti * BM, c0 = (ti + t) * BM;
+  const int lane = threadIdx.x % 64, w = threadIdx.x / 64;
+  const int wr   = (w >> 1) * WM, wc = (w & 1) * WM;
+  const int li   = lane % 16, lk = lane / 16;
+  const int sk   = threadIdx.x % BK, sr = threadIdx.x / BK;
+  const double *pa[VPT], *pb[VPT];
+  f64x4 acc[NI][NI];
+
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
+
+  double va[VPT], vb[VPT];
+
+  // rows past n repeat the last one (their products are not stored)
+#pragma unroll
+  for (int q = 0; q < VPT; ++q)
+  {
+    pa[q] = P + (size_t) min (r0 + sr + RPT * q, n - 1) * K;
+    pb[q] = P + (size_t) min (c0 + sr + RPT * q, n - 1) * K;
+  }
+
+  auto load = [&] (int k0) {
+    const int k   = k0 + sk;
+    const bool in = k < K;
+    const int kk  = in ? k : K - 1;
+
+#pragma unroll
+    for (int q = 0; q < VPT; ++q)
+    {
+      va[q] = pa[q][kk];
+      vb[q] = pb[q][kk];
+    }
+
+    if (!in)
+    {
+#pragma unroll
+      for (int q = 0; q < VPT; ++q)
+        va[q] = vb[q] = 0.0;
+    }
+  };
+  auto store = [&] (int b) {
+#pragma unroll
+    for (int q = 0; q < VPT; ++q)
+    {
+      As[b][sr + RPT * q][sk] = va[q];
+      Bs[b][sr + RPT * q][sk] = vb[q];
+    }
+  };
+
+  load (0);
+  store (0);
+  __syncthreads ();
+
+  int cur = 0;
+
+  for (int k0 = 0; k0 < K; k0 += BK)
+  {
+    if (k0 + BK < K)
+      load (k0 + BK);
+
+#pragma unroll
+    for (int ks = 0; ks < BK / 4; ++ks)
+    {
+      double fa[NI], fb[NI];
+
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+      {
+        fa[i] = As[cur][wr + i * 16 + li][4 * ks + lk];
+        fb[i] = Bs[cur][wc + i * 16 + li][4 * ks + lk];
+      }
+
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64 (fa[i], fb[j], acc[i][j], 0, 0, 0);
+    }
+
+    if (k0 + BK < K)
+      store (cur ^ 1);
+
+    cur ^= 1;
+    __syncthreads ();
+  }
+
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+      {
+        const int a = r0 + wr + i * 16 + lk + 4 * r;
+        const int b = c0 + wc + j * 16 + li;
+
+        if (a < n && b < n && a <= b)
+        {
+          M[(size_t) a * n + b] = acc[i][j][r];
+          M[(size_t) b * n + a] = acc[i][j][r];
+        }
+      }
+}
+template <int BM>
 static void
 launch_syrk_mfma (const double *P, int n, int K, int ld, int off, int kb, double *M, hipStream_t s)
 {
@@ -470,21 +554,32 @@ launch_syrk_mfma (const double *P, int n, int K, int ld, int off, int kb, double
   const int grid   = (ntiles + 7) / 8 * 8;
 
   if (ntiles > 0)
-    hipLaunchKernelGGL ((k_syrk_mfma<MODE, BM>), dim3 (grid), dim3 (256), 0, s, P, n, K, ld, off, kb, M, ntiles);
+    hipLaunchKernelGGL ((k_syrk_mfma<BM>), dim3 (grid), dim3 (256), 0, s, P, n, K, ld, off, kb, M, ntiles);
+}
+
+template <int BM>
+static void
+gram_t (const double *AT, int n, int K, double *M, hipStream_t s)
+{
+  const int nt     = (n + BM - 1) / BM;
+  const int ntiles = nt * (nt + 1) / 2;
+
+  hipLaunchKernelGGL (k_gram<BM>, dim3 ((ntiles + 7) / 8 * 8), dim3 (256), 0, s, AT, n, K, M, ntiles);
 }
 
 hipError_t
 launch_gram_nt (const double *AT, int n, int K, double *M, hipStream_t s)
 {
-  // 128-wide tiles reuse each staged operand twice as often; below about
-  // four blocks per CU their tail leaves the chip half idle, and 64-wide
-  // tiles (4x the blocks) balance better
+  // 128-wide tiles reuse each staged operand twice as often; below about ten
+  // blocks per CU their tail leaves the chip half idle, and 64-wide tiles (4x
+  // the blocks) balance better (n = 6000: 4.08 against 3.99 ms, n = 10000: 17.4
+  // against 18.8)
   const int nt128 = (n + 127) / 128;
 
-  if (nt128 * (nt128 + 1) / 2 >= 1024)
-    launch_syrk_mfma<0, 128> (AT, n, K, K, 0, 0, M, s);
+  if (nt128 * (nt128 + 1) / 2 >= 2560)
+    gram_t<128> (AT, n, K, M, s);
   else
-    launch_syrk_mfma<0, 64> (AT, n, K, K, 0, 0, M, s);
+    gram_t<64> (AT, n, K, M, s);
 
   return hipGetLastError ();
 }
@@ -733,9 +828,9 @@ launch_trailing_update (double *S, int np, int K, int off, int kb, hipStream_t s
   const int nt128 = (np - off + 127) / 128;
 
   if (nt128 * (nt128 + 1) / 2 >= 16384)
-    launch_syrk_mfma<1, 128> (S, np, K, np, off, kb, S, s);
+    launch_syrk_mfma<128> (S, np, K, np, off, kb, S, s);
   else
-    launch_syrk_mfma<1, 64> (S, np, K, np, off, kb, S, s);
+    launch_syrk_mfma<64> (S, np, K, np, off, kb, S, s);
 
   return hipGetLastError ();
 }
