@@ -179,6 +179,9 @@ struct nckde
   // pinned host side of the NNLS loop: solution and gradient read-backs (n
   // doubles each), the active list upload (n ints), solve statistics
   nck::HBuf hnnls;
+  // pinned staging of small host-buffer evals; read-backs of the covariance
+  // factorisations (one word per matrix, then the kNN status)
+  nck::HBuf hev, hinfo;
   // flags of the chained triangular sweeps (status word, then the panel
   // flags; flags_words of them zeroed), the last epoch used, the epoch of a
   // chained solve whose status is still to be read, and whether chained
@@ -280,7 +283,7 @@ check_prepared (nckde *h)
 // (ncm_stats_dist_kde.c:344-367): factor nmats matrices of dcov into dU,
 // then repair the failures on the device.
 static int
-factor_batch (nckde *h, const double *dcov, double *dU, double *dlnnorm, size_t nmats)
+factor_batch (nckde *h, const double *dcov, double *dU, double *dlnnorm, size_t nmats, int *knn_status = nullptr)
 {
   const int d          = h->d;
   const double lconst  = (h->kernel == NCKDE_KERNEL_ST) ? st_lnnorm_const (h) : 0.0;
@@ -289,10 +292,24 @@ factor_batch (nckde *h, const double *dcov, double *dU, double *dlnnorm, size_t 
   HIPCHK (h->dinfo.ensure (sizeof (int) * nmats));
   HIPCHK (nck::launch_chol_batched (dcov, dU, h->dinfo.as<int> (), dlnnorm, d, (int) nmats, h->kernel, lconst, s));
 
-  std::vector<int> info (nmats);
+  HIPCHK (h->hinfo.ensure (sizeof (int) * (nmats + 1)));
 
-  HIPCHK (hipMemcpyAsync (info.data (), h->dinfo.p, sizeof (int) * nmats, hipMemcpyDeviceToHost, s));
+  int *info = h->hinfo.as<int> ();
+
+  HIPCHK (hipMemcpyAsync (info, h->dinfo.p, sizeof (int) * nmats, hipMemcpyDeviceToHost, s));
+
+  if (knn_status != nullptr)
+    HIPCHK (hipMemcpyAsync (info + nmats, h->dstatus.p, sizeof (int), hipMemcpyDeviceToHost, s));
+
   HIPCHK (hipStreamSynchronize (s));
+
+  if (knn_status != nullptr)
+  {
+    *knn_status = info[nmats];
+
+    if (*knn_status != 0)
+      return NCKDE_OK;
+  }
 
   std::vector<int> which;
 
@@ -394,7 +411,10 @@ kde_prepare_kernel (nckde *h)
   }
 
   HIPCHK (nck::launch_whiten (h->dX.as<double> (), h->dUg.as<double> (), h->dY.as<double> (), (int) h->n_obs, d, s));
-  HIPCHK (hipStreamSynchronize (s));
+
+  // the VKDE waits at its local factorisations
+  if (h->kind == NCKDE_KDE)
+    HIPCHK (hipStreamSynchronize (s));
 
   return NCKDE_OK;
 }
@@ -453,10 +473,10 @@ vkde_build_cov_array (nckde *h)
   else
     TRY (robust_cov (h, h->cov_type, (int) h->k, h->dknn.as<int> (), (int) h->n_k, h->dcov.as<double> ()));
 
+  // the selection's status comes back with the factorisations'
   int status = 0;
 
-  HIPCHK (hipMemcpyAsync (&status, h->dstatus.p, sizeof (int), hipMemcpyDeviceToHost, s));
-  HIPCHK (hipStreamSynchronize (s));
+  TRY (factor_batch (h, h->dcov.as<double> (), h->dU.as<double> (), h->dlnnorm.as<double> (), h->n_k, &status));
 
   if (status != 0)
   {
@@ -464,7 +484,7 @@ vkde_build_cov_array (nckde *h)
     return NCKDE_ENUMERIC;
   }
 
-  return factor_batch (h, h->dcov.as<double> (), h->dU.as<double> (), h->dlnnorm.as<double> (), h->n_k);
+  return NCKDE_OK;
 }
 
 static int
@@ -483,12 +503,16 @@ refresh_bvec (nckde *h)
   return NCKDE_OK;
 }
 
+// points and results of a host-buffer eval up to this size go through the
+// handle's pinned buffer
+constexpr size_t HOST_STAGE_BYTES = (size_t) 256 << 10;
+
 static int cv_prepare_minimize (nckde *h);
 static int cv_split_fit (nckde *h, const double *m2lnp, double min_m2lnp);
 
 // _ncm_stats_dist_prepare (ncm_stats_dist.c:703-789)
 static int
-do_prepare (nckde *h)
+do_prepare (nckde *h, bool wait)
 {
   const int d = h->d;
 
@@ -544,12 +568,8 @@ do_prepare (nckde *h)
 
   h->href = get_href (h);
 
-  {
-    std::vector<double> w (h->n_k, 1.0 / (1.0 * h->n_k));
-
-    HIPCHK (h->dw.ensure (sizeof (double) * h->n_k));
-    HIPCHK (hipMemcpyAsync (h->dw.p, w.data (), sizeof (double) * h->n_k, hipMemcpyHostToDevice, h->stream));
-  }
+  HIPCHK (h->dw.ensure (sizeof (double) * h->n_k));
+  HIPCHK (nck::launch_fill (h->dw.as<double> (), h->n_k, 1.0 / (1.0 * h->n_k), h->stream));
 
   HIPCHK (h->dTh.ensure (sizeof (double) * h->n_k * h->D));
 
@@ -566,7 +586,11 @@ do_prepare (nckde *h)
 
   TRY (refresh_bvec (h));
   HIPCHK (h->dwcum.ensure (sizeof (double) * (h->n_k + 1)));
-  HIPCHK (hipStreamSynchronize (h->stream));
+  HIPCHK (h->hev.ensure (HOST_STAGE_BYTES));
+
+  // a fit goes on on the same stream
+  if (wait)
+    HIPCHK (hipStreamSynchronize (h->stream));
 
   h->rnorm       = 0.0;
   h->prepared    = true;
@@ -695,12 +719,7 @@ nnls_refine (nckde *h, int n, int np, double *dxo)
   return NCKDE_OK;
 }
 
-// Unconstrained solve on the sorted index list P (ncm_nnls.c:655-706):
-// NORMAL: Cholesky of the normal matrix (refined against A when its pivots
-// are badly spread), else the symmetric solve, else QR on A_P; NORMAL_LU
-// starts at the symmetric solve; QR solves min |1 - A_P x| directly.
-// The solution is scattered into dxo.
-// the pinned NNLS arena: x (n doubles), g (n doubles), P (n ints), 8 stats
+// the pinned NNLS arena: x (n doubles), g (n doubles), P (n ints), 8 stats, r (n_obs doubles)
 static double *
 nnls_hx (nckde *h)
 {
@@ -725,7 +744,14 @@ nnls_hstat (nckde *h)
   return h->hnnls.as<double> () + 2 * h->n_k + (h->n_k + 1) / 2;
 }
 
-// slot of the pinned statistics that receives the chained sweeps' status
+// the residual (n_obs doubles), after the statistics
+static double *
+nnls_hr (nckde *h)
+{
+  return nnls_hstat (h) + 8;
+}
+
+// slot of the pinned statistics that receives the chained sweep's status
 constexpr int TRSV_STATUS_SLOT = 6;
 
 // U x = y with the factor in dS, y in dtv and x in dbs: the flag-chained sweep
@@ -786,62 +812,22 @@ nnls_trsv_failed (nckde *h)
   return failed;
 }
 
+// pivots of the last factorisation, as k_diag_range and the factor leave them
+struct PivotStat
+{
+  int info, pad;
+  double dmax, dmin;
+};
+
+// the symmetric solve and QR rungs (the first one unless the method is QR)
 static int
-nnls_unconstrained (nckde *h, int n, const std::vector<int> &P, double *dxo)
+nnls_lower_rungs (nckde *h, int n, int np, double *dxo)
 {
   hipStream_t s  = h->stream;
-  const int np   = (int) P.size ();
   const int nobs = (int) h->n_obs;
   bool solved    = false;
 
-  if (progress_enabled ())
-  {
-    fprintf (stderr, "nckde nnls: solve on %d of %d columns\n", np, n);
-    fflush (stderr);
-  }
-
-  if (np == 0)
-  {
-    HIPCHK (hipMemsetAsync (dxo, 0, sizeof (double) * n, s));
-    return NCKDE_OK;
-  }
-
-  // the previous upload from the pinned list ended at that solve's read-back
-  std::memcpy (nnls_hP (h), P.data (), sizeof (int) * np);
-  HIPCHK (hipMemcpyAsync (h->dP.p, nnls_hP (h), sizeof (int) * np, hipMemcpyHostToDevice, s));
-
-  if (h->nnls_umethod == NCKDE_NNLS_NORMAL)
-  {
-    struct
-    {
-      int info, pad;
-      double dmax, dmin;
-    } st = {0, 0, 0.0, 0.0};
-
-    HIPCHK (nck::launch_gather_sym (h->dM.as<double> (), n, h->dP.as<int> (), np, h->dS.as<double> (),
-                                    h->dbv.as<double> (), h->dtv.as<double> (), s));
-    HIPCHK (hipMemsetAsync (h->dscal.p, 0, sizeof (int) * 2, s));
-    HIPCHK (h->dpd.ensure (sizeof (double) * nck::potrf_diag_doubles (np)));
-    HIPCHK (nck::launch_potrf (h->dS.as<double> (), np, h->dtv.as<double> (), h->dscal.as<int> (),
-                               h->dpd.as<double> (), s));
-    HIPCHK (nck::launch_diag_range (h->dS.as<double> (), np, h->dscal.as<double> () + 1, s));
-    HIPCHK (hipMemcpyAsync (nnls_hstat (h), h->dscal.p, sizeof (st), hipMemcpyDeviceToHost, s));
-    HIPCHK (hipStreamSynchronize (s));
-    std::memcpy (&st, nnls_hstat (h), sizeof (st));
-
-    if (st.info == 0)
-    {
-      TRY (nnls_backward (h, np, s));
-      h->nnls_rungs[0]++;
-
-      if (h->nnls_refine > 0 && st.dmax * st.dmax >= REFINE_PIVOT_RATIO * st.dmin * st.dmin)
-        TRY (nnls_refine (h, n, np, dxo));
-
-      solved = true;
-    }
-  }
-
-  if (!solved && h->nnls_umethod != NCKDE_NNLS_QR)
+  if (h->nnls_umethod != NCKDE_NNLS_QR)
   {
     int info = 0;
 
@@ -878,6 +864,93 @@ nnls_unconstrained (nckde *h, int n, const std::vector<int> &P, double *dxo)
   return NCKDE_OK;
 }
 
+// copies the n solution entries to the pinned arena and waits
+static int
+nnls_read_x (nckde *h, int n, const double *dxo)
+{
+  HIPCHK (hipMemcpyAsync (nnls_hx (h), dxo, sizeof (double) * n, hipMemcpyDeviceToHost, h->stream));
+  HIPCHK (hipStreamSynchronize (h->stream));
+
+  return NCKDE_OK;
+}
+
+// Unconstrained solve on the sorted index list P (ncm_nnls.c:655-706), its
+// solution in dxo and in the pinned arena.  NORMAL: Cholesky of the normal
+// matrix (refined against A when its pivots are badly spread), else the
+// symmetric solve, else QR on A_P; NORMAL_LU starts at the symmetric solve; QR
+// solves min |1 - A_P x| directly.  The Cholesky rung is read back once, the factor's status
+// beside the solution: the backward sweep of a failed factor runs on what is
+// there (it ends all the same) and the next rung replaces its result.  retry
+// is set when a chained sweep gave up.
+static int
+nnls_unconstrained (nckde *h, int n, const std::vector<int> &P, double *dxo, bool &retry)
+{
+  hipStream_t s = h->stream;
+  const int np  = (int) P.size ();
+
+  retry = false;
+
+  if (progress_enabled ())
+  {
+    fprintf (stderr, "nckde nnls: solve on %d of %d columns\n", np, n);
+    fflush (stderr);
+  }
+
+  if (np == 0)
+  {
+    HIPCHK (hipMemsetAsync (dxo, 0, sizeof (double) * n, s));
+    return nnls_read_x (h, n, dxo);
+  }
+
+  // the previous upload from the pinned list ended at that solve's read-back
+  std::memcpy (nnls_hP (h), P.data (), sizeof (int) * np);
+  HIPCHK (hipMemcpyAsync (h->dP.p, nnls_hP (h), sizeof (int) * np, hipMemcpyHostToDevice, s));
+
+  if (h->nnls_umethod == NCKDE_NNLS_NORMAL)
+  {
+    PivotStat st;
+
+    HIPCHK (nck::launch_gather_sym (h->dM.as<double> (), n, h->dP.as<int> (), np, h->dS.as<double> (),
+                                    h->dbv.as<double> (), h->dtv.as<double> (), s));
+    HIPCHK (hipMemsetAsync (h->dscal.p, 0, sizeof (int) * 2, s));
+    HIPCHK (h->dpd.ensure (sizeof (double) * nck::potrf_diag_doubles (np)));
+    HIPCHK (nck::launch_potrf (h->dS.as<double> (), np, h->dtv.as<double> (), h->dscal.as<int> (),
+                               h->dpd.as<double> (), s));
+    HIPCHK (nck::launch_diag_range (h->dS.as<double> (), np, h->dscal.as<double> () + 1, s));
+    HIPCHK (hipMemcpyAsync (nnls_hstat (h), h->dscal.p, sizeof (st), hipMemcpyDeviceToHost, s));
+    TRY (nnls_backward (h, np, s));
+    HIPCHK (nck::launch_scatter (h->dbs.as<double> (), h->dP.as<int> (), np, n, dxo, s));
+    TRY (nnls_read_x (h, n, dxo));
+    std::memcpy (&st, nnls_hstat (h), sizeof (st));
+
+    if (st.info == 0)
+    {
+      h->nnls_rungs[0]++;
+
+      if (nnls_trsv_failed (h))
+      {
+        retry = true;
+        return NCKDE_OK;
+      }
+
+      if (h->nnls_refine > 0 && st.dmax * st.dmax >= REFINE_PIVOT_RATIO * st.dmin * st.dmin)
+      {
+        TRY (nnls_refine (h, n, np, dxo));
+        HIPCHK (nck::launch_scatter (h->dbs.as<double> (), h->dP.as<int> (), np, n, dxo, s));
+        TRY (nnls_read_x (h, n, dxo));
+      }
+
+      return NCKDE_OK;
+    }
+
+    h->trsv_pending = 0;
+  }
+
+  TRY (nnls_lower_rungs (h, n, np, dxo));
+
+  return nnls_read_x (h, n, dxo);
+}
+
 // _ncm_nnls_solve_feasible (ncm_nnls.c:728-751)
 static int
 nnls_feasible (nckde *h, int n, std::vector<char> &inP, double *dxo, std::vector<double> &x, int max_remove)
@@ -892,13 +965,13 @@ nnls_feasible (nckde *h, int n, std::vector<char> &inP, double *dxo, std::vector
       if (inP[a])
         P.push_back (a);
 
-    TRY (nnls_unconstrained (h, n, P, dxo));
-    HIPCHK (hipMemcpyAsync (nnls_hx (h), dxo, sizeof (double) * n, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK (hipStreamSynchronize (h->stream));
+    bool retry;
 
-    // a chained triangular solve that gave up: the same solve again with
+    TRY (nnls_unconstrained (h, n, P, dxo, retry));
+
+    // a chained triangular sweep that gave up: the same solve again with
     // one launch per panel
-    if (nnls_trsv_failed (h))
+    if (retry)
       continue;
 
     std::memcpy (x.data (), nnls_hx (h), sizeof (double) * n);
@@ -987,7 +1060,7 @@ nnls_solve (nckde *h)
   HIPCHK (h->dscal.ensure (64));
   HIPCHK (h->dref.ensure (sizeof (double) * 3 * n));
   HIPCHK (h->dcolv.ensure (sizeof (double) * n));
-  HIPCHK (h->hnnls.ensure (sizeof (double) * (2 * (size_t) n + ((size_t) n + 1) / 2 + 8)));
+  HIPCHK (h->hnnls.ensure (sizeof (double) * (2 * (size_t) n + ((size_t) n + 1) / 2 + 8 + (size_t) nobs)));
 
   // M = A^T A, b = A^T f (the QR method works on A alone, ncm_nnls.c:795-797)
   if (h->nnls_umethod != NCKDE_NNLS_QR)
@@ -1051,6 +1124,7 @@ nnls_solve (nckde *h)
       if (rnorm - lrnorm > rnorm * reltol)
       {
         P = Ptry;
+        x = xt;
         HIPCHK (hipMemcpyAsync (h->dx.p, h->dxt.p, sizeof (double) * n, hipMemcpyDeviceToDevice, s));
         HIPCHK (hipMemcpyAsync (h->dr.p, h->drt.p, sizeof (double) * nobs, hipMemcpyDeviceToDevice, s));
         rnorm = lrnorm;
@@ -1074,12 +1148,11 @@ nnls_solve (nckde *h)
   h->rnorm = rnorm;
 
   // the fit's final solution, gradient and residual (diagnostic peek)
-  h->nnls_x.resize (n);
-  h->nnls_r.resize (nobs);
+  h->nnls_x = x;
   h->nnls_g = g;
-  HIPCHK (hipMemcpyAsync (h->nnls_x.data (), h->dx.p, sizeof (double) * n, hipMemcpyDeviceToHost, s));
-  HIPCHK (hipMemcpyAsync (h->nnls_r.data (), h->dr.p, sizeof (double) * nobs, hipMemcpyDeviceToHost, s));
+  HIPCHK (hipMemcpyAsync (nnls_hr (h), h->dr.p, sizeof (double) * nobs, hipMemcpyDeviceToHost, s));
   HIPCHK (hipStreamSynchronize (s));
+  h->nnls_r.assign (nnls_hr (h), nnls_hr (h) + nobs);
 
   return NCKDE_OK;
 }
@@ -1090,7 +1163,7 @@ do_prepare_interp (nckde *h, const double *m2lnp, size_t len)
 {
   const double limit = -2.0 * 2.0 * nck::LOG_DBL_EPSILON;
 
-  TRY (do_prepare (h));
+  TRY (do_prepare (h, false));
 
   if (len != h->n_obs)
   {
@@ -1182,19 +1255,19 @@ do_prepare_interp (nckde *h, const double *m2lnp, size_t len)
   HIPCHK (hipMemsetAsync (h->dstatus.p, 0, sizeof (int) * 4, h->stream));
   HIPCHK (nck::launch_shrink (h->dw.as<double> (), (int) h->n_k, h->shrink, h->dstatus.as<int> (), h->stream));
 
-  int status = 0;
+  TRY (refresh_bvec (h));
+  HIPCHK (h->hinfo.ensure (sizeof (int)));
 
-  HIPCHK (hipMemcpyAsync (&status, h->dstatus.p, sizeof (int), hipMemcpyDeviceToHost, h->stream));
+  int *status = h->hinfo.as<int> ();
+
+  HIPCHK (hipMemcpyAsync (status, h->dstatus.p, sizeof (int), hipMemcpyDeviceToHost, h->stream));
   HIPCHK (hipStreamSynchronize (h->stream));
 
-  if (status != 0)
+  if (*status != 0)
   {
     set_error ("_ncm_stats_dist_prepare_interp: total weight is not positive.");
     return NCKDE_ENUMERIC;
   }
-
-  TRY (refresh_bvec (h));
-  HIPCHK (hipStreamSynchronize (h->stream));
 
   return NCKDE_OK;
 }
@@ -1470,9 +1543,12 @@ fp64_nsplit (const nckde *h, size_t m, int prec)
 
   // up to 2048 points: a split's kernels run one after the other, so splits go
   // down to 4 kernels while the grid stays below 2048 blocks (n = 1000, d = 4:
-  // one point 41 -> 35 us; at 10000 points the larger merge costs more)
+  // one point 41 -> 35 us; at 10000 points the larger merge costs more).  A KDE
+  // split whitens its points first, the work of about d / 2 kernels.
+  const int kmin = (h->kind == NCKDE_KDE) ? std::max (4, h->d / 2) : 4;
+
   if (m <= 2048)
-    maxs = std::max (maxs, std::min ((int) ((h->n_k + 3) / 4), 2048 / nblk));
+    maxs = std::max (maxs, std::min ((int) ((h->n_k + kmin - 1) / kmin), 2048 / nblk));
 
   return std::max (1, std::min (nsplit, maxs));
 }
@@ -1858,6 +1934,27 @@ eval_host (nckde *h, const double *X, size_t m, size_t ld, double *out, int prec
   }
 
   HIPCHK (h->dXe.ensure (sizeof (double) * m * d));
+
+  // small calls: the points go through a pinned buffer, and the merge writes
+  // its m results into it, so that neither direction waits for a staged copy
+  // of pageable memory (one point 35 -> 25 us)
+  if (m * (size_t) (d + 1) * sizeof (double) <= HOST_STAGE_BYTES)
+  {
+    HIPCHK (h->hev.ensure (HOST_STAGE_BYTES));
+
+    double *hx = h->hev.as<double> (), *ho = hx + m * d;
+
+    for (size_t p = 0; p < m; ++p)
+      std::memcpy (hx + p * d, X + p * ld, sizeof (double) * d);
+
+    HIPCHK (hipMemcpyAsync (h->dXe.p, hx, sizeof (double) * m * d, hipMemcpyHostToDevice, h->stream));
+    TRY (eval_device (h, h->dXe.as<double> (), m, ho, precision, linear, h->stream));
+    HIPCHK (hipStreamSynchronize (h->stream));
+    std::memcpy (out, ho, sizeof (double) * m);
+
+    return NCKDE_OK;
+  }
+
   HIPCHK (h->dout.ensure (sizeof (double) * m));
 
   if (ld == (size_t) d)
@@ -3009,7 +3106,7 @@ nckde_prepare (nckde *h)
   TRY (check_handle (h));
   std::lock_guard<std::mutex> lk (h->mtx);
 
-  return do_prepare (h);
+  return do_prepare (h, true);
 }
 
 int
@@ -3312,14 +3409,23 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
     groups[g].push_back (i);
   }
 
+  // every group is queued on its own stream before the first result is waited
+  // for: a group's kernels run under the next one's point copies; the argument
+  // tables and block offsets stay alive until the streams are done
+  std::vector<std::vector<nck::MixedArgs>> gargs (groups.size ());
+  std::vector<std::vector<int>> gblock0 (groups.size ());
+
   for (size_t g = 0; g < groups.size (); ++g)
   {
     const std::vector<size_t> &mem = groups[g];
     nckde *h0                      = hs[mem[0]];
     hipStream_t S                  = h0->stream;
     const int nseg                 = (int) mem.size ();
-    std::vector<nck::MixedArgs> args (nseg);
-    std::vector<int> block0 (2 * (nseg + 1), 0);
+    std::vector<nck::MixedArgs> &args = gargs[g];
+    std::vector<int> &block0          = gblock0[g];
+
+    args.resize (nseg);
+    block0.assign (2 * (nseg + 1), 0);
 
     for (int k = 0; k < nseg; ++k)
     {
@@ -3365,12 +3471,15 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
     HIPCHK (hipMemcpyAsync (dblock0, block0.data (), sizeof (int) * block0.size (), hipMemcpyHostToDevice, S));
     HIPCHK (nck::launch_eval_mixed_multi (args[0].f.DP, h0->kernel, dargs, dblock0, nseg, block0[nseg],
                                           block0[2 * nseg + 1], S));
+  }
 
-    for (int k = 0; k < nseg; ++k)
-      HIPCHK (hipMemcpyAsync (out[mem[k]], hs[mem[k]]->dout.p, sizeof (double) * m[mem[k]], hipMemcpyDeviceToHost,
-                              S));
+  for (const std::vector<size_t> &mem : groups)
+  {
+    hipStream_t S = hs[mem[0]]->stream;
 
-    // the argument table and block offsets stay alive until S is done
+    for (size_t i : mem)
+      HIPCHK (hipMemcpyAsync (out[i], hs[i]->dout.p, sizeof (double) * m[i], hipMemcpyDeviceToHost, S));
+
     HIPCHK (hipStreamSynchronize (S));
   }
 

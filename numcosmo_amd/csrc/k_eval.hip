@@ -335,7 +335,7 @@ launch_f32_b2 (const double *b, double bref, int n, float *b2f, hipStream_t s)
 // l + L, ...; the lanes' maxima and sums combine as a tree in LDS, so the
 // result depends on nsplit and L only.  The reads of the partials bound it:
 // 8 lanes keep 256-byte rows coalesced over 32 points and are used from 2048
-// points on; below, 64 lanes (256 up to 64 points) shorten the serial walk
+// points on; below, 64 lanes (256 up to 256 points) shorten the serial walk
 // over the splits, which one lane per point ran in 66 us at m = 6400.
 __global__ void __launch_bounds__ (256)
 k_eval_merge (EvalArgs a, int L)
@@ -504,7 +504,7 @@ launch_eval_f64 (const EvalArgs &a, hipStream_t s)
 hipError_t
 launch_eval_merge (const EvalArgs &a, hipStream_t s)
 {
-  const int L = (a.m >= 2048) ? 8 : (a.m > 64) ? 64 : 256;
+  const int L = (a.m >= 2048) ? 8 : (a.m > 256) ? 64 : 256;
 
   hipLaunchKernelGGL (k_eval_merge, dim3 ((a.m + 256 / L - 1) / (256 / L)), dim3 (256), 0, s, a, L);
 

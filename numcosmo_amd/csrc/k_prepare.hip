@@ -1372,6 +1372,24 @@ launch_kde_factors (const double *Y, int nk, int d, int D, double *Th, hipStream
   return hipGetLastError ();
 }
 
+__global__ void
+k_fill (double *__restrict__ x, size_t n, double v)
+{
+  const size_t i = blockIdx.x * (size_t) blockDim.x + threadIdx.x;
+
+  if (i < n)
+    x[i] = v;
+}
+
+hipError_t
+launch_fill (double *x, size_t n, double v, hipStream_t s)
+{
+  if (n > 0)
+    hipLaunchKernelGGL (k_fill, dim3 ((unsigned) ((n + 255) / 256)), dim3 (256), 0, s, x, n, v);
+
+  return hipGetLastError ();
+}
+
 // b_i = ln w_i - lnnorm_i (the per-kernel constant of sum0/sum1)
 __global__ void
 k_bvec (const double *__restrict__ w, const double *__restrict__ lnnorm, int nk, double *__restrict__ b)

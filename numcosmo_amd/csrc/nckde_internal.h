@@ -165,6 +165,7 @@ size_t knn_max_k ();
 hipError_t launch_vkde_factors (const double *U, const double *X, int nk, int d, int D, double *Wp,
                                 double *Th, hipStream_t s);
 hipError_t launch_kde_factors (const double *Y, int nk, int d, int D, double *Th, hipStream_t s);
+hipError_t launch_fill (double *x, size_t n, double v, hipStream_t s);
 hipError_t launch_bvec (const double *w, const double *lnnorm, int nk, double *b, hipStream_t s);
 
 // ---- evaluation (k_eval.hip) --------------------------------------------

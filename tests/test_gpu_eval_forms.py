@@ -112,3 +112,27 @@ def test_mixed_groups(oracle, nu, d, n, m):
     P = np.concatenate([g.normal(size=(m, d)), X[:1], 40.0 * g.normal(size=(1, d))])
     got, ref = sd.eval_m2lnp_batch(P, 1), od.eval_m2lnp_batch(P)
     assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-6
+
+
+@pytest.mark.parametrize("d", [3, 7])
+@pytest.mark.parametrize("extra", [-1, 0, 1])
+def test_host_staging(oracle, d, extra):
+    """Host-buffer evals around the size (256 KiB of points and results) up to
+    which they go through the pinned buffer, packed and with a row stride: each
+    point's value does not depend on the way it came in."""
+    import numcosmo_amd as na
+    from numcosmo_amd._lib import check, lib
+    g = np.random.default_rng(8)
+    X = g.normal(size=(120, d))
+    sd, od = _pair(oracle, 1, 3.0, d, X)
+    m = (256 << 10) // (8 * (d + 1)) + extra
+    wide = g.normal(size=(m, d + 2))
+    P = np.ascontiguousarray(wide[:, :d])
+    got = sd.eval_m2lnp_batch(P, 0)
+    out = np.empty(m)
+    check(lib().nckde_eval_m2lnp(sd._h, wide, m, d + 2, out, 0))
+    assert np.array_equal(got, out)
+    ref = od.eval_m2lnp_batch(P[-50:])
+    assert np.max(np.abs(got[-50:] - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-12
+    # a smaller call afterwards reuses the buffer
+    assert np.max(np.abs(sd.eval_m2lnp_batch(P[:5], 0) - got[:5]) / np.maximum(np.abs(got[:5]), 1.0)) < 1e-12
