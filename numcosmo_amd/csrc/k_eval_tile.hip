@@ -1,7 +1,7 @@
 // k_eval_tile.hip -- FP64 and FP32 eval of the VKDE from 13 dimensions on,
 // with the whitening product on the matrix cores (kde_tile.h).
 //
-// A wave takes 64 (or 32) points and walks its split's kernels; each lane
+// A wave takes 64 points (FP64 above d = 32: 32) and walks its split's kernels; each lane
 // ends a step with the squared norm of one pair and adds its term.  The terms
 // and their two forms are those of k_eval.hip, and so are the partial (max,
 // sum) pairs that k_eval_merge combines.
@@ -136,27 +136,24 @@ k_eval_tile_f32 (EvalArgs a)
   tile.load_points (a.X, p0, a.m, a.d, a.D);
 
   const int lp       = p0 + tile.lane_point ();
-  const int lk       = tile.lane_kernel ();
   const float inv_h2 = (float) a.inv_h2;
   const float kappa  = (float) a.kappa;
   const float inv_nu = (float) (1.0 / a.nu);
   float M            = -INFINITY;
   double S           = 0.0;
 
-  for (int i = i0; i < i1; i += P::KU)
+  static_assert (P::KU == 1, "one kernel per step");
+
+  for (int i = i0; i < i1; ++i)
   {
     const float chi2 = tile.chi2 (a.Wf, a.Th, i, i1) * inv_h2;
-    const bool on    = (P::KU == 1) || (i + lk < i1);
-    const float b2   = a.b2f[on ? i + lk : i];
+    const float b2   = a.b2f[i];
     float lnt;
 
     if (KERNEL == NCKDE_KERNEL_GAUSS)
       lnt = fmaf (-0.5f, chi2, b2);
     else
       lnt = fmaf (kappa, log1pf (chi2 * inv_nu), b2);
-
-    if (!on)
-      lnt = -INFINITY;
 
     if (lnt > M)
     {
@@ -167,17 +164,7 @@ k_eval_tile_f32 (EvalArgs a)
     S += (lnt > -INFINITY) ? (double) expf (lnt - M) : 0.0;
   }
 
-  if (P::KU == 2)
-  {
-    const float Mo  = __shfl_xor (M, 16, 64);
-    const double So = __shfl_xor (S, 16, 64);
-    const float Mx  = fmaxf (M, Mo);
-
-    S = ((M > -INFINITY) ? S * (double) expf (M - Mx) : 0.0) + ((Mo > -INFINITY) ? So * (double) expf (Mo - Mx) : 0.0);
-    M = Mx;
-  }
-
-  if (lp < a.m && lk == 0)
+  if (lp < a.m)
   {
     a.partM[(size_t) blockIdx.y * a.m + lp] = (M > -INFINITY) ? (double) M + a.bref : -INFINITY;
     a.partS[(size_t) blockIdx.y * a.m + lp] = S;
@@ -188,9 +175,9 @@ template <int NK, int KERNEL>
 static hipError_t
 tile_t (const EvalArgs &a, hipStream_t s)
 {
-  constexpr int PTS = PairTile<double, NK>::PTS;
-  const int waves   = (a.m + PTS - 1) / PTS;
-  const int wpb     = (waves < 4) ? waves : 4;
+  const int PTS   = (a.b2f != nullptr) ? PairTile<float, NK>::PTS : PairTile<double, NK>::PTS;
+  const int waves = (a.m + PTS - 1) / PTS;
+  const int wpb   = (waves < 4) ? waves : 4;
   const dim3 grid ((waves + wpb - 1) / wpb, a.nsplit), block (64 * wpb);
 
   if (a.b2f != nullptr)

@@ -85,20 +85,24 @@ tile_swap16 (double a, double b)
   return __hiloint2double ((int) hi[0], (int) lo[0]) + __hiloint2double ((int) hi[1], (int) lo[1]);
 }
 
-// Point tiles per wave: the coordinates take 2 NT NK registers and the
+// Point tiles per wave: the coordinates take 2 NT NK registers and the FP64
 // accumulators 8 NT NRT, so 4 tiles up to d = 32 and 2 above (two waves per
 // SIMD either way).  With 2 tiles a step takes 2 kernels, so that all 64
-// lanes hold a pair in the terms.
+// lanes hold a pair in the terms.  FP32 accumulators take half of that, and
+// an FP32 step half the time of an FP64 one while its fragments of W_i cost the
+// vector L1 the same 16 lines: 4 tiles always (FP32, n = 8000, m = 40000: 28.4
+// against 16.8 ms at d = 64, 15.1 against 8.9-11.7 at d = 40).
+template <typename T>
 constexpr int
 tile_nt (int NK)
 {
-  return (NK <= 8) ? 4 : 2;
+  return (NK <= 8 || sizeof (T) == 4) ? 4 : 2;
 }
 
 template <typename T, int NK>
 struct PairTile
 {
-  static constexpr int NT  = tile_nt (NK);
+  static constexpr int NT  = tile_nt<T> (NK);
   static constexpr int KU  = 4 / NT;            // kernels per step
   static constexpr int NRT = (NK + 3) / 4;      // row tiles
   static constexpr int PTS = 16 * NT;           // points per wave
