@@ -1,12 +1,12 @@
-// k_eval.hip -- FP64 eval_m2lnp / eval for KDE and VKDE.
+// k_eval.hip -- FP64 and FP32 eval_m2lnp / eval for KDE, and for VKDE below 13
+// dimensions (k_eval_tile.hip has the others).
 //
 // One lane per evaluation point; every lane of a block walks the same kernel
 // range, so the kernel factors (packed W_i = U_i^{-T}, centre, b_i) are
 // wave-uniform and come in through scalar loads straight into SGPR operands
 // of the FP64 FMAs.  Per pair (VKDE, padded dim D): D subtractions,
-// D(D+1)/2 FMAs for z = W_i (x - theta_i), D FMAs for |z|^2, one exp (two
-// transcendentals for Student-t).  The log-sum-exp runs online in FP64 with
-// a running maximum.  The kernel range is split over blockIdx.y so that small
+// D(D+1)/2 FMAs for z = W_i (x - theta_i), D FMAs for |z|^2, and the kernel's
+// term in one of the two forms below.  The kernel range is split over blockIdx.y so that small
 // point counts still fill the 256 CUs; partial (max, sum) pairs are merged in
 // split order by k_eval_merge.
 //

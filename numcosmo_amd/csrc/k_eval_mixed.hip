@@ -10,9 +10,10 @@
 // z' is accumulated in FP32 by v_mfma_f32_32x32x16_f16 from three products
 // (A_hi y_hi + A_hi y_lo + A_lo y_hi), with -c_i (stored negated) as the
 // accumulator input.
-// Each 32-row MFMA tile holds 32/DP kernels (DP = padded dimension 4, 8, 16)
-// or one kernel over 1 or 2 row tiles (DP = 32, 64); for DP < 16 the hi/lo
-// operands are packed along K so no K lanes are wasted.
+// Each 32-row MFMA tile holds 32/DP kernels (DP = padded dimension 4, 8), 8 rows
+// of four kernels (DP = 16) or 16 rows of two (DP = 32, 64), with K up to the
+// diagonal of the triangular factors; for DP < 16 and the upper rows of DP = 16
+// the hi/lo operands are packed along K so no K lanes are wasted.
 //
 // The kernel sum runs on the VALU in base 2: lnt2 = log2(e) lnt - b_ref with
 //   Gauss  lnt2 = q_i |z'|^2 + b2_i,               q_i = -log2(e) / (2 s_i^2)
