@@ -61,7 +61,9 @@ k_lu_init (double *__restrict__ S, int np, double *__restrict__ colv)
 }
 
 // pivot of column k: first maximum of colv[k..np); info = k + 1 when it is
-// zero; otherwise rows k and piv are swapped (columns k..np) with b
+// zero or there is none (a column of NaN, where the search keeps its start
+// value np, one row past the matrix); otherwise rows k and piv are swapped
+// (columns k..np) with b
 __global__ void __launch_bounds__ (1024)
 k_lu_pivot (double *__restrict__ S, int np, int k, double *__restrict__ b, const double *__restrict__ colv,
             int *__restrict__ info)
@@ -111,7 +113,7 @@ k_lu_pivot (double *__restrict__ S, int np, int k, double *__restrict__ b, const
   const double amax = rv[0];
   const int piv     = ri[0];
 
-  if (amax == 0.0)
+  if (amax == 0.0 || piv >= np)
   {
     if (tid == 0)
       *info = k + 1;
