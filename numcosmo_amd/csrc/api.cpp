@@ -3100,13 +3100,26 @@ nckde_reset (nckde *h)
   return NCKDE_OK;
 }
 
+// A prepare or fit that ends with an error leaves nothing queued on the
+// handle's stream: the getters read through the null stream, which does not
+// wait for it, and the copies in flight read the host sample, which the caller
+// may change next.
+static int
+settled (nckde *h, int status)
+{
+  if (status != NCKDE_OK)
+    (void) hipStreamSynchronize (h->stream);
+
+  return status;
+}
+
 int
 nckde_prepare (nckde *h)
 {
   TRY (check_handle (h));
   std::lock_guard<std::mutex> lk (h->mtx);
 
-  return do_prepare (h, true);
+  return settled (h, do_prepare (h, true));
 }
 
 int
@@ -3125,7 +3138,7 @@ nckde_prepare_interp (nckde *h, const double *m2lnp, size_t n)
   for (unsigned &c : h->nnls_rungs)
     c = 0;
 
-  return do_prepare_interp (h, m2lnp, n);
+  return settled (h, do_prepare_interp (h, m2lnp, n));
 }
 
 int

@@ -41,3 +41,31 @@ def test_nan_m2lnp(umethod, n):
     twin.add_obs_array(X)
     twin.prepare_interp(m2)
     assert np.array_equal(sd.peek_weights(), twin.peek_weights())
+
+
+def test_refused_length_leaves_uniform_weights():
+    """m2lnp of the wrong length: the sample is prepared, with equal weights,
+    and they are there when the call returns, also while other work holds the
+    GPU (the getter reads on another stream than the prepare writes on)."""
+    import torch
+    from numcosmo_amd._lib import lib
+    g = np.random.default_rng(7)
+    n, d = 600, 4
+    X = g.normal(size=(n, d))
+    m2 = np.sum(X * X, 1)
+    sd = _new(0, 0, d)
+    sd.add_obs_array(X)
+    A = torch.randn(4096, 4096, device="cuda")
+    side = torch.cuda.Stream()
+    for _ in range(20):
+        sd.prepare_interp(m2)
+        w = np.empty(n)
+        assert not np.allclose(sd.peek_weights(), 1.0 / n)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            for _ in range(10):
+                A @ A
+        assert lib().nckde_prepare_interp(sd._h, np.append(m2, 0.0), n + 1) == EINVAL
+        assert lib().nckde_get_weights(sd._h, w) == 0
+        assert np.array_equal(w, np.full(n, 1.0 / n))
+    torch.cuda.synchronize()
