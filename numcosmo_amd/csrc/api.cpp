@@ -487,18 +487,36 @@ vkde_build_cov_array (nckde *h)
   return NCKDE_OK;
 }
 
+// queues b and the terms made of it; with status, neither is written when
+// *status (on the device) is not 0
 static int
-refresh_bvec (nckde *h)
+queue_bvec (nckde *h, const int *status)
 {
   HIPCHK (h->db.ensure (sizeof (double) * h->n_k));
   HIPCHK (nck::launch_bvec (h->dw.as<double> (), (h->kind == NCKDE_VKDE) ? h->dlnnorm.as<double> () : nullptr,
-                            (int) h->n_k, h->db.as<double> (), h->stream));
+                            (int) h->n_k, h->db.as<double> (), status, h->stream));
   HIPCHK (h->dterm.ensure (sizeof (double) * (h->n_k + 1)));
-  HIPCHK (nck::launch_eval_terms (h->db.as<double> (), (int) h->n_k, h->kernel, h->dterm.as<double> (), h->stream));
+  HIPCHK (nck::launch_eval_terms (h->db.as<double> (), (int) h->n_k, h->kernel, h->dterm.as<double> (), status,
+                                  h->stream));
+
+  return NCKDE_OK;
+}
+
+// what was made from the weights before is out of date
+static void
+weights_changed (nckde *h)
+{
   h->wcum_ready    = false;
   h->mixed_b_ready = false;
   h->f32_b_ready   = false;
   h->graph_gen++;
+}
+
+static int
+refresh_bvec (nckde *h)
+{
+  TRY (queue_bvec (h, nullptr));
+  weights_changed (h);
 
   return NCKDE_OK;
 }
@@ -1255,7 +1273,9 @@ do_prepare_interp (nckde *h, const double *m2lnp, size_t len)
   HIPCHK (hipMemsetAsync (h->dstatus.p, 0, sizeof (int) * 4, h->stream));
   HIPCHK (nck::launch_shrink (h->dw.as<double> (), (int) h->n_k, h->shrink, h->dstatus.as<int> (), h->stream));
 
-  TRY (refresh_bvec (h));
+  // weights without a positive total leave b as the prepare made it (equal
+  // weights), so that the handle still evaluates after the error
+  TRY (queue_bvec (h, h->dstatus.as<int> ()));
   HIPCHK (h->hinfo.ensure (sizeof (int)));
 
   int *status = h->hinfo.as<int> ();
@@ -1268,6 +1288,8 @@ do_prepare_interp (nckde *h, const double *m2lnp, size_t len)
     set_error ("_ncm_stats_dist_prepare_interp: total weight is not positive.");
     return NCKDE_ENUMERIC;
   }
+
+  weights_changed (h);
 
   return NCKDE_OK;
 }

@@ -400,10 +400,14 @@ k_eval_merge (EvalArgs a, int L)
 // Student-t term_i = exp (b_i - bref), Gauss term_i = (b_i - bref) log2 e;
 // term[n] = bref.  One block: the arrays are n doubles.
 __global__ void __launch_bounds__ (1024)
-k_eval_terms (const double *__restrict__ b, int n, int kernel, double *__restrict__ term)
+k_eval_terms (const double *__restrict__ b, int n, int kernel, double *__restrict__ term,
+              const int *__restrict__ status)
 {
   __shared__ double red[1024];
   double M = -INFINITY;
+
+  if (status != nullptr && *status != 0)
+    return;
 
   for (int i = threadIdx.x; i < n; i += 1024)
     M = fmax (M, b[i]);
@@ -433,9 +437,9 @@ k_eval_terms (const double *__restrict__ b, int n, int kernel, double *__restric
 }
 
 hipError_t
-launch_eval_terms (const double *b, int n, int kernel, double *term, hipStream_t s)
+launch_eval_terms (const double *b, int n, int kernel, double *term, const int *status, hipStream_t s)
 {
-  hipLaunchKernelGGL (k_eval_terms, dim3 (1), dim3 (1024), 0, s, b, n, kernel, term);
+  hipLaunchKernelGGL (k_eval_terms, dim3 (1), dim3 (1024), 0, s, b, n, kernel, term, status);
 
   return hipGetLastError ();
 }

@@ -1392,20 +1392,21 @@ launch_fill (double *x, size_t n, double v, hipStream_t s)
 
 // b_i = ln w_i - lnnorm_i (the per-kernel constant of sum0/sum1)
 __global__ void
-k_bvec (const double *__restrict__ w, const double *__restrict__ lnnorm, int nk, double *__restrict__ b)
+k_bvec (const double *__restrict__ w, const double *__restrict__ lnnorm, int nk, double *__restrict__ b,
+        const int *__restrict__ status)
 {
   const long i = blockIdx.x * (long) blockDim.x + threadIdx.x;
 
-  if (i >= nk)
+  if (i >= nk || (status != nullptr && *status != 0))
     return;
 
   b[i] = log (w[i]) - (lnnorm ? lnnorm[i] : 0.0);
 }
 
 hipError_t
-launch_bvec (const double *w, const double *lnnorm, int nk, double *b, hipStream_t s)
+launch_bvec (const double *w, const double *lnnorm, int nk, double *b, const int *status, hipStream_t s)
 {
-  hipLaunchKernelGGL (k_bvec, dim3 ((nk + 255) / 256), dim3 (256), 0, s, w, lnnorm, nk, b);
+  hipLaunchKernelGGL (k_bvec, dim3 ((nk + 255) / 256), dim3 (256), 0, s, w, lnnorm, nk, b, status);
 
   return hipGetLastError ();
 }

@@ -166,7 +166,8 @@ hipError_t launch_vkde_factors (const double *U, const double *X, int nk, int d,
                                 double *Th, hipStream_t s);
 hipError_t launch_kde_factors (const double *Y, int nk, int d, int D, double *Th, hipStream_t s);
 hipError_t launch_fill (double *x, size_t n, double v, hipStream_t s);
-hipError_t launch_bvec (const double *w, const double *lnnorm, int nk, double *b, hipStream_t s);
+// status: NULL, or a device word; nothing is written when it is not 0
+hipError_t launch_bvec (const double *w, const double *lnnorm, int nk, double *b, const int *status, hipStream_t s);
 
 // ---- evaluation (k_eval.hip) --------------------------------------------
 struct EvalArgs
@@ -202,8 +203,8 @@ hipError_t launch_eval_f64 (const EvalArgs &a, hipStream_t s);
 hipError_t launch_f32_factors (const double *Wp, size_t count, float *Wf, hipStream_t s);
 hipError_t launch_f32_b2 (const double *b, double bref, int n, float *b2f, hipStream_t s);
 hipError_t launch_eval_merge (const EvalArgs &a, hipStream_t s);
-// term: n + 1 doubles (the last one max_i b_i)
-hipError_t launch_eval_terms (const double *b, int n, int kernel, double *term, hipStream_t s);
+// term: n + 1 doubles (the last one max_i b_i); status as in launch_bvec
+hipError_t launch_eval_terms (const double *b, int n, int kernel, double *term, const int *status, hipStream_t s);
 // nu + d when the Student-t kernel is an integer power of rsqrt (1 + chi2 /
 // nu) that half_power takes, else 0
 inline int

@@ -69,3 +69,31 @@ def test_refused_length_leaves_uniform_weights():
         assert lib().nckde_get_weights(sd._h, w) == 0
         assert np.array_equal(w, np.full(n, 1.0 / n))
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind,kernel", [(0, 0), (1, 1), (1, 0)])
+@pytest.mark.parametrize("why", ["nan", "zero"])
+def test_no_positive_weight_keeps_the_prepared_density(kind, kernel, why):
+    """A fit whose weights have no positive total (NaN in m2lnp; a bandwidth so
+    wide that every kernel underflows to 0) ends with an error, and the handle
+    evaluates as its prepare left it, with equal weights, in every precision."""
+    g = np.random.default_rng(9)
+    n, d = 300, 3
+    X = g.normal(size=(n, d))
+    m2 = np.sum(X * X, 1)
+    P = g.normal(size=(3000, d))
+    sd, twin = _new(kind, kernel, d), _new(kind, kernel, d)
+    for o in (sd, twin):
+        if why == "zero":
+            o.set_over_smooth(1e110)
+        o.add_obs_array(X)
+    if why == "nan":
+        m2[n // 2] = np.nan
+    with pytest.raises(NckdeError) as e:
+        sd.prepare_interp(m2)
+    assert e.value.status == ENUMERIC
+    twin.prepare()
+    for precision in (0, 1, 2):
+        got, ref = sd.eval_m2lnp_batch(P, precision), twin.eval_m2lnp_batch(P, precision)
+        assert np.all(np.isfinite(ref))
+        assert np.array_equal(got, ref)
