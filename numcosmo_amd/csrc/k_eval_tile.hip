@@ -12,6 +12,17 @@
 namespace nck
 {
 
+// the (max, sum) pairs of a point's two lanes, one per kernel of a step
+__device__ inline void
+join_halves (double &M, double &S)
+{
+  const double Mo = __shfl_xor (M, 16, 64), So = __shfl_xor (S, 16, 64);
+  const double Mx = fmax (M, Mo);
+
+  S = ((M > -INFINITY) ? S * exp (M - Mx) : 0.0) + ((Mo > -INFINITY) ? So * exp (Mo - Mx) : 0.0);
+  M = Mx;
+}
+
 template <int NK, int KERNEL>
 __global__ void __launch_bounds__ (256)
 k_eval_tile (EvalArgs a)
@@ -35,21 +46,34 @@ k_eval_tile (EvalArgs a)
   double M     = -INFINITY, S = 0.0;
   bool done    = false;
 
-  // against the common reference max_i b_i, without logarithm or running
-  // maximum (see k_eval_f64)
-  if (KERNEL == NCKDE_KERNEL_GAUSS || a.pw > 0)
+  // the fast forms of k_eval_f64
+  if (KERNEL == NCKDE_KERNEL_GAUSS)
+  {
+    Pow2Sum<P::KU == 1> sum;
+
+    for (int i = i0; i < i1; i += P::KU)
+    {
+      const double chi2 = tile.chi2 (a.Wp, a.Th, i, i1);
+      const bool on     = (P::KU == 1) || (i + lk < i1);
+      const double t    = fma (chi2, a.fc, a.term[on ? i + lk : i]);
+
+      sum.add (on ? t : -1.0e300);
+    }
+
+    sum.result (*a.tref, M, S);
+
+    if (P::KU == 2)
+      join_halves (M, S);
+
+    done = (S > 0.0) && (S < INFINITY);
+  }
+  else if (a.pw > 0)
   {
     for (int i = i0; i < i1; i += P::KU)
     {
       const double chi2 = tile.chi2 (a.Wp, a.Th, i, i1);
       const bool on     = (P::KU == 1) || (i + lk < i1);
-      const double tm   = a.term[on ? i + lk : i];
-      double e;
-
-      if (KERNEL == NCKDE_KERNEL_GAUSS)
-        e = exp2_f64 (fma (chi2, a.fc, tm));
-      else
-        e = tm * half_power (fma (chi2, a.fc, 1.0), a.pw);
+      const double e    = a.term[on ? i + lk : i] * half_power (fma (chi2, a.fc, 1.0), a.pw);
 
       S += on ? e : 0.0;
     }
@@ -66,7 +90,7 @@ k_eval_tile (EvalArgs a)
   {
     double Mg = -INFINITY, Sg = 0.0;
 
-    for (int i = i0; i < i1; i += P::KU)
+    for (int i = some_weight (a.b, i0, i1) ? i0 : i1; i < i1; i += P::KU)
     {
       const double chi2 = tile.chi2 (a.Wp, a.Th, i, i1) * a.inv_h2;
       const bool on     = (P::KU == 1) || (i + lk < i1);
@@ -93,13 +117,7 @@ k_eval_tile (EvalArgs a)
     }
 
     if (P::KU == 2)
-    {
-      const double Mo = __shfl_xor (Mg, 16, 64), So = __shfl_xor (Sg, 16, 64);
-      const double Mx = fmax (Mg, Mo);
-
-      Sg = ((Mg > -INFINITY) ? Sg * exp (Mg - Mx) : 0.0) + ((Mo > -INFINITY) ? So * exp (Mo - Mx) : 0.0);
-      Mg = Mx;
-    }
+      join_halves (Mg, Sg);
 
     if (!done)
     {

@@ -51,31 +51,112 @@ half_power (double u, int p)
   return t;
 }
 
-// 2^t for t <= 0 (0 below the subnormals): t = n + f with f in [-1/2, 1/2],
-// the Taylor polynomial of exp (f ln 2) to order 13 (remainder below
-// (ln 2 / 2)^14 / 14! = 5e-18), and the exponent by ldexp.
-__device__ inline double
-exp2_f64 (double t)
+// a whole number as an int, saturated (-2^31 for -inf, 0 for NaN); outside its
+// range the conversion of the language is undefined
+__device__ inline int
+saturated_int (double n)
 {
-  const double n = rint (t);
-  const double x = (t - n) * 0.69314718055994530941723212145817657;
-  double p       = 1.0 / 6227020800.0;
+  int k;
 
-  p = fma (p, x, 1.0 / 479001600.0);
-  p = fma (p, x, 1.0 / 39916800.0);
-  p = fma (p, x, 1.0 / 3628800.0);
-  p = fma (p, x, 1.0 / 362880.0);
-  p = fma (p, x, 1.0 / 40320.0);
-  p = fma (p, x, 1.0 / 5040.0);
-  p = fma (p, x, 1.0 / 720.0);
-  p = fma (p, x, 1.0 / 120.0);
-  p = fma (p, x, 1.0 / 24.0);
-  p = fma (p, x, 1.0 / 6.0);
-  p = fma (p, x, 0.5);
-  p = fma (p, x, 1.0);
-  p = fma (p, x, 1.0);
+  __asm__ ("v_cvt_i32_f64 %0, %1" : "=v" (k) : "v" (n));
 
-  return ldexp (p, (int) n);
+  return k;
+}
+
+// S 2^R = the sum of the 2^t that were added (t <= 0), R a whole number up to
+// 512 below the largest t: one integer comparison per term instead of a
+// maximum and a rescaling, and no term is lost beside a sum of about 1 or more,
+// wherever the terms lie.  Terms below 2^-(2^30) add nothing; -inf and NaN make
+// the sum NaN.
+//
+// 2^t is taken as 2^n exp (f ln 2), n = rint (t), f in [-1/2, 1/2].  The
+// polynomial 1 + x + x^2 g (x) interpolates g = (exp (x) - 1 - x) / x^2 at the
+// Chebyshev nodes of |x| <= ln 2 / 2; its largest error is 3.4e-19 (a Taylor
+// polynomial needs one order more for 5e-18).
+//
+// The rescaling is a wave-uniform branch, kept one by the empty asm: as the
+// selects that the compiler makes of it every term pays for it (16 % at d = 4).
+// LATE: after the addition, which leaves a step's code in one piece (d = 16, n =
+// 4000, m = 20000: 0.79 ms, 0.82 with the branch first), but holds both sums,
+// which at d = 64 spills (7.9 against 6.0 ms).
+template <bool LATE>
+struct Pow2Sum
+{
+  int R    = -(1 << 30);
+  double S = 0.0;
+
+  __device__ inline void
+  add (double t)
+  {
+    const double n = rint (t);
+    const double x = (t - n) * 0.69314718055994530941723212145817657;
+    int k          = saturated_int (n);
+    double p       = 0x1.1f72fc730b4ffp-29;
+
+    p = fma (p, x, 0x1.af4ddd84882fep-26);
+    p = fma (p, x, 0x1.27e4db67b4303p-22);
+    p = fma (p, x, 0x1.71de02375656cp-19);
+    p = fma (p, x, 0x1.a01a01a6d7808p-16);
+    p = fma (p, x, 0x1.a01a01abe62ddp-13);
+    p = fma (p, x, 0x1.6c16c16c162d6p-10);
+    p = fma (p, x, 0x1.11111111100dfp-7);
+    p = fma (p, x, 0x1.5555555555556p-5);
+    p = fma (p, x, 0x1.5555555555557p-3);
+    p = fma (p, x, 0.5);
+    p = fma (p, x, 1.0);
+    p = fma (p, x, 1.0);
+
+    const double Sn = LATE ? S + ldexp (p, k - R) : 0.0;
+
+    if (__any (k - R > 512))
+    {
+      __asm__ ("" : "+v" (k));
+
+      const bool up = k - R > 512;
+      const int r   = up ? k : R;
+
+      S = (LATE && !up) ? Sn : ldexp (S, R - r) + (LATE ? p : 0.0);
+      R = r;
+    }
+    else if (LATE)
+    {
+      S = Sn;
+    }
+
+    if (!LATE)
+      S += ldexp (p, k - R);
+  }
+
+  // the sum as s exp (m - ref): with m = ref itself, which every split shares and
+  // the merge of the splits takes without an exponential, while s stays well
+  // within range (R <= 0, since no t is above 0)
+  __device__ inline void
+  result (double ref, double &m, double &s) const
+  {
+    if (R > -900)
+    {
+      m = ref;
+      s = ldexp (S, R);
+    }
+    else
+    {
+      m = (S > 0.0) ? fma ((double) R, 0.69314718055994530941723212145817657, ref) : -INFINITY;
+      s = S;
+    }
+  }
+};
+
+// a kernel of [i0, i1) with a weight: a range of zero weights (b = -inf) has
+// no terms to form
+__device__ inline bool
+some_weight (const double *__restrict__ b, int i0, int i1)
+{
+  bool any = false;
+
+  for (int i = i0; i < i1 && !any; ++i)
+    any = (b[i] != -INFINITY);
+
+  return any;
 }
 
 // Rows of a packed factor that a padded dimension D <= 12 may not need: rows

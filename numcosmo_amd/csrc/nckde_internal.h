@@ -191,8 +191,8 @@ struct EvalArgs
   const float *Wf = nullptr, *b2f = nullptr;
   double bref     = 0.0;
 };
-// Smallest sum of a split that the fast form of the FP64 terms may return:
-// above it the terms lost to underflow (under 1e-308) cannot be seen.
+// Smallest sum of a split that the fast form of the FP64 Student-t terms may
+// return: above it the terms lost to underflow (under 1e-308) cannot be seen.
 constexpr double EVAL_FAST_FLOOR = 1.0e-250;
 // dimension from which the VKDE's per-pair products run on the matrix cores
 // (k_eval_tile.hip, k_im_tile.hip)
