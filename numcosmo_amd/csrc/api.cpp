@@ -179,6 +179,9 @@ struct nckde
   // pinned host side of the NNLS loop: solution and gradient read-backs (n
   // doubles each), the active list upload (n ints), solve statistics
   nck::HBuf hnnls;
+  // set while the split fit evaluates its residuals: Gauss terms in the general
+  // form (cv_split_fit)
+  bool general_terms = false;
   // pinned staging of small host-buffer evals; read-backs of the covariance
   // factorisations (one word per matrix, then the kNN status)
   nck::HBuf hev, hinfo;
@@ -1771,7 +1774,7 @@ eval_device (nckde *h, const double *dX, size_t m, double *dout, int precision, 
     return eval_fp64_ws (h, dX, m, dout, linear, s, nullptr, precision == NCKDE_PREC_FP32);
   };
 
-  if (!h->graphs || h->profiling || s == nullptr)
+  if (!h->graphs || h->profiling || s == nullptr || h->general_terms)
     return run ();
 
   return eval_graph (h, dX, m, dout, precision, linear, s, run);
@@ -1916,6 +1919,7 @@ eval_fp64_ws (nckde *h, const double *dX, size_t m, double *dout, int linear, hi
   a.term          = h->dterm.as<double> ();
   a.tref          = h->dterm.as<double> () + h->n_k;
   a.pw            = nck::half_power_of (h->kernel, h->nu, h->d);
+  a.general       = h->general_terms;
   a.fc            = (h->kernel == NCKDE_KERNEL_GAUSS) ? -0.5 * nck::LOG2E_D * a.inv_h2 : a.inv_h2 / h->nu;
 
   if (f32)
@@ -2318,7 +2322,16 @@ cv_split_fit (nckde *h, const double *m2lnp, double min_m2lnp)
 
     TRY (cv_fit_at (h, lp, min_m2lnp, rn));
     TRY (refresh_bvec (h));
-    TRY (cv_eval_rows (h, 0, no, v));
+
+    // the fit's weights hold zeros.  Near a singular interpolation matrix the
+    // path of the fit depends on the rounding of these residuals: they keep the
+    // form (logarithms, running maximum) that the fit is tested with.
+    h->general_terms = true;
+
+    const int st = cv_eval_rows (h, 0, no, v);
+
+    h->general_terms = false;
+    TRY (st);
 
     double fn2 = 0.0;
 

@@ -128,13 +128,16 @@ k_eval_f64 (EvalArgs a)
 
   if (KERNEL == NCKDE_KERNEL_GAUSS)
   {
-    Pow2Sum<true> sum;
+    if (!a.general)
+    {
+      Pow2Sum<true> sum;
 
-    for (int i = i0; i < i1; ++i)
-      sum.add (fma (chi2_of (i), a.fc, a.term[i]));
+      for (int i = i0; i < i1; ++i)
+        sum.add (fma (chi2_of (i), a.fc, a.term[i]));
 
-    sum.result (*a.tref, M, S);
-    done = (S > 0.0) && (S < INFINITY);
+      sum.result (*a.tref, M, S);
+      done = (S > 0.0) && (S < INFINITY);
+    }
   }
   else if (a.pw > 0)
   {

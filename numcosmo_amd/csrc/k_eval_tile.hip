@@ -49,23 +49,26 @@ k_eval_tile (EvalArgs a)
   // the fast forms of k_eval_f64
   if (KERNEL == NCKDE_KERNEL_GAUSS)
   {
-    Pow2Sum<P::KU == 1> sum;
-
-    for (int i = i0; i < i1; i += P::KU)
+    if (!a.general)
     {
-      const double chi2 = tile.chi2 (a.Wp, a.Th, i, i1);
-      const bool on     = (P::KU == 1) || (i + lk < i1);
-      const double t    = fma (chi2, a.fc, a.term[on ? i + lk : i]);
+      Pow2Sum<P::KU == 1> sum;
 
-      sum.add (on ? t : -1.0e300);
+      for (int i = i0; i < i1; i += P::KU)
+      {
+        const double chi2 = tile.chi2 (a.Wp, a.Th, i, i1);
+        const bool on     = (P::KU == 1) || (i + lk < i1);
+        const double t    = fma (chi2, a.fc, a.term[on ? i + lk : i]);
+
+        sum.add (on ? t : -1.0e300);
+      }
+
+      sum.result (*a.tref, M, S);
+
+      if (P::KU == 2)
+        join_halves (M, S);
+
+      done = (S > 0.0) && (S < INFINITY);
     }
-
-    sum.result (*a.tref, M, S);
-
-    if (P::KU == 2)
-      join_halves (M, S);
-
-    done = (S > 0.0) && (S < INFINITY);
   }
   else if (a.pw > 0)
   {

@@ -128,20 +128,23 @@ struct Pow2Sum
   }
 
   // the sum as s exp (m - ref): with m = ref itself, which every split shares and
-  // the merge of the splits takes without an exponential, while s stays well
-  // within range (R <= 0, since no t is above 0)
+  // the merge of the splits takes without an exponential, while s is well
+  // within range (R <= 0, since no t is above 0), else with s near 1, so that
+  // the larger of two m is that of the larger sum
   __device__ inline void
   result (double ref, double &m, double &s) const
   {
-    if (R > -900)
+    const int e = __builtin_amdgcn_frexp_exp (S);   // 0 for 0, inf and NaN
+
+    if (R + e > -900)
     {
       m = ref;
       s = ldexp (S, R);
     }
     else
     {
-      m = (S > 0.0) ? fma ((double) R, 0.69314718055994530941723212145817657, ref) : -INFINITY;
-      s = S;
+      m = (S > 0.0) ? fma ((double) (R + e), 0.69314718055994530941723212145817657, ref) : -INFINITY;
+      s = ldexp (S, -e);
     }
   }
 };

@@ -187,6 +187,7 @@ struct EvalArgs
   const double *term = nullptr, *tref = nullptr;
   double fc          = 0.0;
   int pw             = 0;
+  int general        = 0;          // Gauss terms in the general form
   // FP32 rung (b2f != NULL): FP32 factors (VKDE), b_i - bref in FP32
   const float *Wf = nullptr, *b2f = nullptr;
   double bref     = 0.0;

@@ -74,6 +74,21 @@ def test_separated_modes(oracle, kind, d, order, m):
     assert _err(sd.eval_m2lnp_batch(P), od.eval_m2lnp_batch(P)) < 1e-12
 
 
+@pytest.mark.parametrize("kind,d", [(0, 1), (1, 1), (0, 4), (1, 4), (1, 16), (1, 36)])
+def test_outwards(oracle, kind, d):
+    """Points from the centre to 1e5 widths out: sums against max b, between it
+    and what underflows, and far below, in splits whose first kernel lies
+    hundreds of powers of two under their nearest one."""
+    g = np.random.default_rng(d)
+    X = g.standard_t(4.0, size=(12 * d + 200, d))
+    X[::7] *= 3.0
+    sd, od = _pair(oracle, kind, d, X)
+    u = g.normal(size=(400, d))
+    P = u / np.linalg.norm(u, axis=1)[:, None] * np.exp(np.linspace(np.log(0.1), np.log(1e5), 400))[:, None]
+    assert _err(sd.eval_m2lnp_batch(P), od.eval_m2lnp_batch(P)) < 1e-12
+    assert _err(np.array([sd.eval_m2lnp(p) for p in P[::40]]), od.eval_m2lnp_batch(P[::40])) < 1e-12
+
+
 @pytest.mark.parametrize("d,m", [(4, 20000), (16, 2048)])
 def test_time_does_not_depend_on_the_weights_or_the_modes(d, m):
     """Each split once: 1.3 times the plain sample's kernel time at most.  The
