@@ -1722,15 +1722,49 @@ static int eval_graph (nckde *h, const double *dX, size_t m, double *dout, int p
                        const Run &run);
 
 // Mixed evals that the FP64 form finishes sooner: its two launches against the
-// mixed form's five, and splits of few kernels against its groups (measured
-// per call at n = 600 / 3000 / 20000: d = 6, m = 64: 9 / 12 / 22 us against 16 /
-// 19 / 42; d = 16, m = 256: 13 / 28 / 89 against 23 / 30 / 86; d = 40, m = 256:
-// 25 / 64 / 314 against 74 / - / 378; d = 3, m = 128: 9 / 16 / 35 against 17 / 17 /
-// 29).  The factors are built all the same.
+// mixed form's five, and splits of few kernels against its groups.  The lines
+// lie where the two forms took the same time in 13000 evals of 65 to 3000
+// points (d = 2 ... 64, n = 200 ... 50000, KDE and VKDE, Gauss, Student-t with
+// integer and other nu).  FP64 time grows with the points in steps of a wave (64
+// points, 32 at D >= 48) and with the kernel term (the general form, which a nu
+// that is not a whole number takes, costs most at small d; Gauss most at large
+// d), and above 2048 points its splits are longer; mixed time hardly grows up to
+// 256 points.  Microseconds, FP64 / mixed:
+//   d = 8,  m = 128:  nu = 3    36 / 39 (n = 20000);  nu = 2.5  26 / 23 (6000)
+//   d = 16, m = 256:  nu = 3    13 / 23 (600), 56 / 47 (8000), 89 / 86 (20000);  nu = 2.5  49 / 39 (6000)
+//   d = 40, m = 256:  nu = 3    314 / 378 (20000);  Gauss  597 / 486 (27000)
+//   d = 64, m = 128:  nu = 5    258 / 328 (12700);  nu = 2.5  1.3 times mixed (17000)
+//   d = 64, m = 256:  nu = 5    201 / 246 (5100), 1.4 times mixed (12700);  Gauss  936 / 440 (20000)
+// The factors are built all the same.
 static bool
 mixed_small (const nckde *h, size_t m)
 {
-  return m <= 64 || (h->d > 4 && m <= 128) || (h->d >= 13 && m <= 256) || m * h->n_k <= 750000;
+  const size_t n     = h->n_k;
+  const int D        = h->D;
+  const bool gauss   = h->kernel == NCKDE_KERNEL_GAUSS;
+  const bool general = !gauss && nck::half_power_of (h->kernel, h->nu, h->d) == 0;
+  size_t few         = (D == 4 || (general && D == 8)) ? 64 : (D <= 12) ? 128 : 256;          // points
+  size_t pairs       = (!general || D > 12) ? 750000 : (D == 12) ? 600000 : 480000;
+
+  // (a KDE's FP64 pair takes d products, not d^2 / 2: no limit by n)
+  if (h->kind == NCKDE_VKDE)
+  {
+    const bool wide = general && h->d > 56;
+
+    if (D == 16)
+      few = general ? 128 : (n > 5000 && n <= 14000) ? 192 : 256;
+    else if ((D == 32 && general && n > 18000) || (D == 48 && (general || gauss) && n > 8000))
+      few = 128;
+    else if (D == 64 && n > (size_t) (wide ? 4000 : 8000))
+      few = (wide && n > 14000) ? 64 : 128;
+
+    if (D == 16 && general)
+      pairs = 520000;
+    else if ((D == 24 || D == 32) && m > 640)
+      pairs = 500000;
+  }
+
+  return m <= 64 || m <= few || (m * n <= pairs && (m <= 2048 || (D == 4 && !general)));
 }
 
 static int
