@@ -2464,6 +2464,19 @@ struct Reader
 
 const char SER_MAGIC[8] = {'N', 'C', 'K', 'D', 'E', '0', '2', '\0'};
 
+// Streams that are waited for when a call leaves early: what is queued on them
+// reads host tables of the call and the buffers of handles it has locked.
+struct Drain
+{
+  std::vector<hipStream_t> streams;
+
+  ~Drain ()
+  {
+    for (hipStream_t s : streams)
+      (void) hipStreamSynchronize (s);
+  }
+};
+
 } // namespace
 
 extern "C" {
@@ -3400,8 +3413,10 @@ nckde_eval_m2lnp_device_noalloc (nckde *h, const double *dX, size_t m, double *d
 // Mixed-precision evals of handles that share the MFMA dimension and kernel
 // type run as one launch per pass over a segment table; every segment's
 // blocks compute what the handle's own eval computes, so the results are
-// bit-identical to separate calls.  Other precisions, and handles whose
-// mixed factors fall back to FP64, run one by one.
+// bit-identical to separate calls.  Other precisions, and handles whose mixed
+// eval runs in FP64 (factors that fell back, few points) or takes a pilot pass,
+// run one by one, each waited for (six sessions of 8 to 128 points, d = 8 and 16:
+// 160 to 215 us, 310 fused).
 int
 nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *m, const size_t *ld,
                         double *const *out, size_t count, int precision)
@@ -3496,6 +3511,7 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
   // tables and block offsets stay alive until the streams are done
   std::vector<std::vector<nck::MixedArgs>> gargs (groups.size ());
   std::vector<std::vector<int>> gblock0 (groups.size ());
+  Drain queued;
 
   for (size_t g = 0; g < groups.size (); ++g)
   {
@@ -3508,6 +3524,7 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
 
     args.resize (nseg);
     block0.assign (2 * (nseg + 1), 0);
+    queued.streams.push_back (S);
 
     for (int k = 0; k < nseg; ++k)
     {
@@ -3564,6 +3581,8 @@ nckde_eval_m2lnp_multi (nckde *const *hs, const double *const *X, const size_t *
 
     HIPCHK (hipStreamSynchronize (S));
   }
+
+  queued.streams.clear ();
 
   return NCKDE_OK;
 }
