@@ -77,17 +77,14 @@ template <int NK, int KERNEL>
 static hipError_t
 imt_t (const IMArgs &a, hipStream_t s)
 {
-  static int resident = 0;
-
-  if (resident == 0)
-  {
+  static const int resident = [] {
     int dev = 0, ncu = 0, nb = 0;
 
     (void) hipGetDevice (&dev);
     (void) hipDeviceGetAttribute (&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb, k_im_tile<NK, KERNEL>, 256, 0);
-    resident = (nb > 0 ? nb : 1) * (ncu > 0 ? ncu : 1);
-  }
+    return (nb > 0 ? nb : 1) * (ncu > 0 ? ncu : 1);
+  }();
 
   constexpr int PB = 4 * PairTile<double, NK>::PTS;
   const int bx     = (a.n_obs + PB - 1) / PB;

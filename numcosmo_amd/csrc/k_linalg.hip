@@ -148,17 +148,14 @@ template <int D, int KERNEL, int KIND>
 static hipError_t
 im_t (const IMArgs &a, hipStream_t s)
 {
-  static int resident = 0;
-
-  if (resident == 0)
-  {
+  static const int resident = [] {
     int dev = 0, ncu = 0, nb = 0;
 
     (void) hipGetDevice (&dev);
     (void) hipDeviceGetAttribute (&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb, k_build_IM<D, KERNEL, KIND>, 256, 0);
-    resident = (nb > 0 ? nb : 1) * (ncu > 0 ? ncu : 1);
-  }
+    return (nb > 0 ? nb : 1) * (ncu > 0 ? ncu : 1);
+  }();
 
   const int bx     = (a.n_obs + 255) / 256;
   const int total0 = bx * ((2048 + bx - 1) / bx);
@@ -545,6 +542,7 @@ k_gram (const double *__restrict__ P, int n, int K, double *__restrict__ M, int 
         }
       }
 }
+
 template <int BM>
 static void
 launch_syrk_mfma (const double *P, int n, int K, int ld, int off, int kb, double *M, hipStream_t s)
@@ -1150,17 +1148,14 @@ k_trsv_chain (const double *__restrict__ S, int np, const double *__restrict__ r
 int
 trsv_chain_max_panels ()
 {
-  static int cap = -1;
-
-  if (cap < 0)
-  {
+  static const int cap = [] {
     int dev = 0, ncu = 0, nb = 0;
 
     (void) hipGetDevice (&dev);
     (void) hipDeviceGetAttribute (&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     (void) hipOccupancyMaxActiveBlocksPerMultiprocessor (&nb, k_trsv_chain, 64, 0);
-    cap = (nb > 0 && ncu > 0) ? nb * ncu : 0;
-  }
+    return (nb > 0 && ncu > 0) ? nb * ncu : 0;
+  }();
 
   return cap;
 }
@@ -1180,148 +1175,6 @@ hipError_t
 launch_mirror_lower (double *S, int np, hipStream_t s)
 {
   hipLaunchKernelGGL (k_mirror_lower, dim3 ((np + 255) / 256, np), dim3 (256), 0, s, S, np);
-
-  return hipGetLastError ();
-}
-
-// --------------------------------------------------------------------------
-// Fallback when the normal matrix is not numerically SPD (the reference's
-// dsysv path, ncm_nnls.c:574-605): Gaussian elimination with partial
-// pivoting (first maximum) on the symmetrised matrix, one 1024-thread block.
-// --------------------------------------------------------------------------
-__global__ void __launch_bounds__ (1024)
-k_lu_solve (double *__restrict__ S, int np, double *__restrict__ b, int *__restrict__ info)
-{
-  __shared__ double rv[1024];
-  __shared__ int ri[1024];
-  const int tid = threadIdx.x;
-
-  for (size_t e = tid; e < (size_t) np * np; e += 1024)
-  {
-    const int i = (int) (e / np), j = (int) (e % np);
-
-    if (j < i)
-      S[e] = S[(size_t) j * np + i];
-  }
-
-  __syncthreads ();
-
-  for (int k = 0; k < np; ++k)
-  {
-    double best = -1.0;
-    int bi      = np;
-
-    for (int i = k + tid; i < np; i += 1024)
-    {
-      const double v = fabs (S[(size_t) i * np + k]);
-
-      if (v > best)
-      {
-        best = v;
-        bi   = i;
-      }
-    }
-
-    rv[tid] = best;
-    ri[tid] = bi;
-    __syncthreads ();
-
-    for (int o = 512; o > 0; o >>= 1)
-    {
-      if (tid < o)
-      {
-        const double v2 = rv[tid + o];
-        const int i2    = ri[tid + o];
-
-        if (v2 > rv[tid] || (v2 == rv[tid] && i2 < ri[tid]))
-        {
-          rv[tid] = v2;
-          ri[tid] = i2;
-        }
-      }
-
-      __syncthreads ();
-    }
-
-    const double amax = rv[0];
-    const int piv     = ri[0];
-
-    __syncthreads ();
-
-    if (amax == 0.0)
-    {
-      if (tid == 0)
-        *info = k + 1;
-
-      return;
-    }
-
-    if (piv != k)
-    {
-      for (int j = tid; j < np; j += 1024)
-      {
-        const double t          = S[(size_t) k * np + j];
-        S[(size_t) k * np + j]   = S[(size_t) piv * np + j];
-        S[(size_t) piv * np + j] = t;
-      }
-
-      if (tid == 0)
-      {
-        const double t = b[k];
-
-        b[k]   = b[piv];
-        b[piv] = t;
-      }
-    }
-
-    __syncthreads ();
-
-    const int rows = np - k - 1;
-
-    for (size_t e = tid; e < (size_t) rows * (rows + 1); e += 1024)
-    {
-      const int i    = k + 1 + (int) (e / (rows + 1));
-      const int jj   = (int) (e % (rows + 1));
-      const double l = S[(size_t) i * np + k] / S[(size_t) k * np + k];
-
-      if (jj < rows)
-      {
-        const int j = k + 1 + jj;
-
-        S[(size_t) i * np + j] = S[(size_t) i * np + j] - l * S[(size_t) k * np + j];
-      }
-      else
-      {
-        b[i] = b[i] - l * b[k];
-      }
-    }
-
-    __syncthreads ();
-  }
-
-  for (int i = np - 1; i >= 0; --i)
-  {
-    if (tid == 0)
-    {
-      double t = b[i];
-
-      for (int j = i + 1; j < np; ++j)
-        t = t - S[(size_t) i * np + j] * b[j];
-
-      b[i] = t / S[(size_t) i * np + i];
-    }
-
-    __syncthreads ();
-  }
-
-  if (tid == 0)
-    *info = 0;
-}
-
-hipError_t
-launch_lu_solve (double *S, int np, double *b, int *info, hipStream_t s)
-{
-  hipLaunchKernelGGL (k_lu_solve, dim3 (1), dim3 (1024), 0, s, S, np, b, info);
 
   return hipGetLastError ();
 }

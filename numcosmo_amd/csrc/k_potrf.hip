@@ -35,7 +35,7 @@ struct StepArgs
   int *info;             // first failing pivot + 1 (LAPACK), else 0
   double *Ud;            // factored diagonal block (row-major 64 x 64, upper)
   double *b;             // right-hand side: y = U^{-T} b in place
-  int npb, nrb, row_end, ntiles;
+  int npb, nrb, ntiles;
 };
 
 // double broadcast from lane `src` (wave-uniform)
@@ -705,7 +705,6 @@ potrf_step (double *S, int np, int kb, bool upd, int row_end, double *b, int *in
   a.b       = b;
   a.npb     = (rest > 0) ? (rest + CH_NB - 1) / CH_NB : 1;
   a.nrb     = (kb > 0 && rest > 0) ? (rest + 255) / 256 : 0;
-  a.row_end = row_end;
   a.ntiles  = 0;
 
   if (upd && rest > 0 && row_end > off)
@@ -738,7 +737,11 @@ launch_potrf (double *S, int np, double *b, int *info, double *diagbuf, hipStrea
       for (int kp = kb; kp < ke; kp += CH_NB)
         potrf_step (S, np, kp, kp > kb, ke, b, info, diagbuf, s);
 
-      launch_trailing_update (S, np, SP_NB, ke, kb, s);
+      const hipError_t e = launch_trailing_update (S, np, SP_NB, ke, kb, s);
+
+      if (e != hipSuccess)
+        return e;
+
       kb = ke;
       continue;
     }

@@ -318,7 +318,6 @@ hipError_t launch_trsv_pair (const double *S, int np, double *b, double *tmp, hi
 int trsv_chain_max_panels ();
 hipError_t launch_trsv_chain (const double *S, int np, const double *y, double *x, unsigned *flags, unsigned epoch,
                               hipStream_t s);
-hipError_t launch_lu_solve (double *S, int np, double *b, int *info, hipStream_t s);
 hipError_t launch_trsv_backward (const double *S, int np, double *y, double *x, hipStream_t s);
 hipError_t launch_mirror_lower (double *S, int np, hipStream_t s);
 // k_nnls.hip: the symmetric-solve and QR rungs, refinement helpers
