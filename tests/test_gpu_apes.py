@@ -74,6 +74,8 @@ def test_apes_bounds_respected():
 
 
 def test_apes_mixed_precision_stationary():
+    """A run that asks for mixed precision (its few walkers evaluate in FP64
+    there; the mixed form runs in test_apes_step_at_full_size)."""
     _say("[apes] stationary dim=3 ST3 kernel, mixed-precision transition densities")
     tgt, s = _run(3, 1, 60, precision=1, seed=5)
     chain = s.chain[10:]
@@ -113,7 +115,9 @@ def test_apes_moves_match_oracle(oracle, ktype, precision, rtol):
     each half-step starts from (rebuilt from the initial sample and the
     recorded decisions), the two transition densities
     (ncm_fit_esmcmc_walker_apes.c:819-881), the exploration countdown
-    (:815-816) and the acceptance rule (:884-919)."""
+    (:815-816) and the acceptance rule (:884-919).  The third case asks for mixed
+    precision; with this few walkers it evaluates in FP64 (the mixed form runs in
+    test_apes_step_at_full_size)."""
     import math
     from numcosmo_amd.apes import APES, InterpolationKernel
     dim, nw, steps, expl, rw, os_, lf = 2, 120, 4, 3, 0.25, 0.2, 0.2

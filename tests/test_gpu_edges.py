@@ -65,12 +65,16 @@ def test_ragged_point_counts(oracle, kind, kernel, d, n, lf):
     X = g.normal(size=(n, d))
     sd, od = _pair(oracle, kind, kernel, d, X, local_frac=lf)
     for m in (1, 2, 31, 33, 127, 129, 255, 257, 511, 513, 1025):
-        Y = g.normal(size=(m, d)) * 1.5
+        # mixed evals of few points run in FP64: the mixed form takes 4096 more
+        # (whole tiles and blocks), so that the same partial ones are left
+        Y = g.normal(size=(4096 + m, d)) * 1.5
         ref = od.eval_m2lnp_batch(Y)
-        e64 = _rel(sd.eval_m2lnp_batch(Y, precision=0), ref).max()
-        emx = _rel(sd.eval_m2lnp_batch(Y, precision=1), ref).max()
+        e64 = _rel(sd.eval_m2lnp_batch(Y[-m:], precision=0), ref[-m:]).max()
+        mix = sd.eval_m2lnp_batch(Y, precision=1)
+        emx = _rel(mix, ref).max()
         assert e64 <= 1e-12, (m, e64)
         assert emx <= 1e-6, (m, emx)
+        assert not np.array_equal(mix, sd.eval_m2lnp_batch(Y, precision=0)), m
     _say(f"   kind={kind} d={d}: ragged m ok")
 
 
@@ -78,15 +82,26 @@ def test_ragged_point_counts(oracle, kind, kernel, d, n, lf):
                                                 (1, ST, 8, 21, 0.6), (0, GAUSS, 16, 19, None)])
 def test_padding_kernels(oracle, kind, kernel, d, n, lf):
     """Kernel counts that are not a multiple of the kernels per MFMA group
-    (8 at d <= 4, 4 at d <= 8, 2 at d <= 16): the padding kernels carry zero
-    weight and change no result."""
+    (8 at d <= 4, 4 at d <= 16, 2 above): the padding kernels carry zero
+    weight and change no result.  As many points as the mixed form needs to
+    run (750000 pairs at d <= 4, 2048 points above)."""
     g = np.random.default_rng(20 + n)
     X = g.normal(size=(n, d))
     sd, od = _pair(oracle, kind, kernel, d, X, local_frac=lf)
-    Y = np.vstack([X, g.normal(size=(300, d))])
+    # a probe above its tolerance (five kernels: 6e-7) would send the handle to
+    # FP64: the mixed form runs all the same here, within ten times the probe's
+    # error where that is above the bar
+    sd.set_mixed_tolerance(1e-3)
+    bar = max(1e-6, 10.0 * sd.get_mixed_check()[0])
+    m = 2049 if d > 4 else 750000 // n + 1
+    Y = np.vstack([X, g.normal(size=(m, d))])
     ref = od.eval_m2lnp_batch(Y)
-    assert _rel(sd.eval_m2lnp_batch(Y, precision=0), ref).max() <= 1e-12
-    assert _rel(sd.eval_m2lnp_batch(Y, precision=1), ref).max() <= 1e-6
+    e64 = sd.eval_m2lnp_batch(Y, precision=0)
+    emx = sd.eval_m2lnp_batch(Y, precision=1)
+    assert _rel(e64, ref).max() <= 1e-12
+    _say(f"   probe bar {bar:.1e}, mixed error {_rel(emx, ref).max():.1e}")
+    assert _rel(emx, ref).max() <= bar
+    assert not np.array_equal(emx, e64)
     u = np.concatenate([[0.0, np.nextafter(1.0, 0.0)], g.uniform(size=200)])
     np.testing.assert_array_equal(sd.kernel_choose_batch(u), [od.kernel_choose(p) for p in u])
 
@@ -96,7 +111,13 @@ def test_one_dimension(oracle, kind, kernel, nu):
     g = np.random.default_rng(30 + kind)
     X = g.standard_t(4.0, size=(200, 1))
     sd, od = _pair(oracle, kind, kernel, 1, X, nu=nu)
-    Y = np.linspace(-30.0, 30.0, 401).reshape(-1, 1)
+    sd.set_mixed_tolerance(1e-3)   # as in test_padding_kernels
+    bar = max(1e-6, 10.0 * sd.get_mixed_check()[0])
+    Y = np.linspace(-30.0, 30.0, 4001).reshape(-1, 1)   # 800200 pairs: the mixed form runs
     ref = od.eval_m2lnp_batch(Y)
-    assert _rel(sd.eval_m2lnp_batch(Y, precision=0), ref).max() <= 1e-12
-    assert _rel(sd.eval_m2lnp_batch(Y, precision=1), ref).max() <= 1e-6
+    e64 = sd.eval_m2lnp_batch(Y, precision=0)
+    emx = sd.eval_m2lnp_batch(Y, precision=1)
+    assert _rel(e64, ref).max() <= 1e-12
+    _say(f"   probe bar {bar:.1e}, mixed error {_rel(emx, ref).max():.1e}")
+    assert _rel(emx, ref).max() <= bar
+    assert not np.array_equal(emx, e64)

@@ -100,18 +100,28 @@ def test_interpolation_matrix(oracle, nu, d, n):
 
 
 @pytest.mark.parametrize("nu", [0.0, 3.0])
-@pytest.mark.parametrize("d,n", [(3, 129), (8, 130), (9, 131), (12, 161), (16, 162), (16, 163), (17, 321), (32, 322),
-                                 (33, 323), (48, 324), (64, 325), (64, 1027)])
-@pytest.mark.parametrize("m", [1, 33, 800])
-def test_mixed_groups(oracle, nu, d, n, m):
-    """Mixed evals with kernel counts that leave part of a group, and point
-    counts around the 32-point tiles: 1e-6 relative, the bar of the mixed path."""
-    g = np.random.default_rng(d * n + m)
+@pytest.mark.parametrize("d,n", [(2, 1601), (3, 1604), (4, 1607), (5, 1601), (8, 1603), (9, 1601), (12, 1602),
+                                 (16, 1601), (16, 1603), (17, 1601), (32, 1603), (33, 1601), (48, 1603), (49, 1601),
+                                 (64, 1603)])
+def test_mixed_groups(oracle, nu, d, n):
+    """Mixed evals with kernel counts that leave part of a group (8, 4, 4, 2, 2
+    kernels), and point counts around the 32-point tiles and the blocks of 512
+    (768 at d = 9 to 16): 1e-6 relative, the bar of the mixed path.  More than 800
+    points of 1600 kernels, since fewer run in FP64."""
+    g = np.random.default_rng(d * n)
     X = g.normal(size=(n, d))
     sd, od = _pair(oracle, 1, nu, d, X)
-    P = np.concatenate([g.normal(size=(m, d)), X[:1], 40.0 * g.normal(size=(1, d))])
-    got, ref = sd.eval_m2lnp_batch(P, 1), od.eval_m2lnp_batch(P)
-    assert np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0)) < 1e-6
+    # the probe of the riskiest kernels (1e-6 at d = 64) would send the handle to FP64
+    sd.set_mixed_tolerance(1e-5)
+    assert not sd.get_mixed_check()[1]
+    P = np.concatenate([g.normal(size=(1601, d)), X[:1], 40.0 * g.normal(size=(1, d))])
+    ref = od.eval_m2lnp_batch(P)
+    for m in (800, 801, 831, 1024, 1025, 1536, 1537, 1603):
+        Q, r = P[-m:], ref[-m:]
+        got = sd.eval_m2lnp_batch(Q, 1)
+        # the mixed form ran: the FP64 one gives the FP64 eval's results to the bit
+        assert not np.array_equal(got, sd.eval_m2lnp_batch(Q, 0))
+        assert np.max(np.abs(got - r) / np.maximum(np.abs(r), 1.0)) < 1e-6
 
 
 @pytest.mark.parametrize("d", [3, 7])

@@ -297,8 +297,9 @@ def test_nearpd_path_rank_deficient(gpu, oracle, d, n, local_frac, maxiter):
 
 
 MIXED_CASES = [
-    # kernel, d (padded MFMA dim 4, 8, 16, 32, 64), n, nu
-    (GAUSS, 3, 700, 0.0),
+    # kernel, d (padded MFMA dim 4, 8, 16, 32, 64), n (with 1000 points, enough
+    # for the mixed form to run), nu
+    (GAUSS, 3, 801, 0.0),
     (ST, 8, 1500, 3.0),
     (ST, 12, 900, 1.0),
     (GAUSS, 16, 2000, 0.0),
@@ -335,6 +336,8 @@ def test_eval_m2lnp_mixed_precision(gpu, oracle, kind, kernel, d, n, nu):
     _say(f"   mixed max rel err {err.max():.3e} p99 {np.quantile(err, 0.99):.3e}")
     assert np.all(np.isfinite(got))
     assert err.max() <= 1e-6
+    # (unless its probe sent the handle to FP64) the mixed form ran
+    assert sd.get_mixed_check()[1] or not np.array_equal(got, sd.eval_m2lnp_batch(Xe, gpu.Precision.FP64))
     # batch composition does not change a point's result beyond the tolerance
     alone = sd.eval_m2lnp_batch(Xe[10:11], gpu.Precision.MIXED)
     assert abs(alone[0] - got[10]) <= 1e-6 * max(abs(ref[10]), 1.0)
@@ -394,10 +397,11 @@ def test_mixed_after_refit_uses_new_weights(gpu, oracle):
     X = tgt.draw(g, n)
     sd, od = _pair(gpu, oracle, 1, ST, d, X, 3.0)
     sd.prepare()
-    Xe = tgt.draw(g, 300)
+    Xe = tgt.draw(g, 1000)         # 800000 pairs: the mixed form runs
     a = sd.eval_m2lnp_batch(Xe, gpu.Precision.MIXED)
     sd.prepare_interp(tgt.m2lnp(X))
     b = sd.eval_m2lnp_batch(Xe, gpu.Precision.MIXED)
+    assert not np.array_equal(b, sd.eval_m2lnp_batch(Xe, gpu.Precision.FP64))
     od.prepare()
     od.set_weights(sd.peek_weights())
     ref = od.eval_m2lnp_batch(Xe)
