@@ -568,13 +568,13 @@ gram_t (const double *AT, int n, int K, double *M, hipStream_t s)
 hipError_t
 launch_gram_nt (const double *AT, int n, int K, double *M, hipStream_t s)
 {
-  // 128-wide tiles reuse each staged operand twice as often; below about ten
+  // 128-wide tiles reuse each staged operand twice as often; below about seven
   // blocks per CU their tail leaves the chip half idle, and 64-wide tiles (4x
-  // the blocks) balance better (n = 6000: 4.08 against 3.99 ms, n = 10000: 17.4
-  // against 18.8)
+  // the blocks) balance better (128- against 64-wide: n = 5800 4.3 / 4.0 ms, 6400
+  // and 7000 equal, 7600 8.1 / 8.6, 8800 11.8 / 13.4, 10000 18.3 / 19.5)
   const int nt128 = (n + 127) / 128;
 
-  if (nt128 * (nt128 + 1) / 2 >= 2560)
+  if (nt128 * (nt128 + 1) / 2 >= 1800)
     gram_t<128> (AT, n, K, M, s);
   else
     gram_t<64> (AT, n, K, M, s);
