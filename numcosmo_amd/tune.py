@@ -48,15 +48,14 @@ def default_nsplit(prec, d, n, m):
     """The library's default rule (api.cpp mixed_nsplit / fp64_nsplit)."""
     if prec == 1:
         DP = _mfma_dim(d)
-        kpt = 1 if DP >= 32 else 32 // DP
-        ngroups = (n + kpt - 1) // kpt
-        ppb = (2 if DP == 64 else (8 if DP == 16 else 4)) * 32 * (8 if DP == 64 else 4)
+        kpt = 8 if DP == 4 else (4 if DP <= 16 else 2)                   # kernels per group
+        ppb = {16: 768}.get(DP, 512)                                     # points per block
+        kmin = 8 if DP >= 32 else 256 // DP                              # kernels per split, at least
         bx = (m + ppb - 1) // ppb
-        ns = (8192 + bx - 1) // bx
-        return max(1, min(ns, max(1, ngroups // 8))), ngroups
+        return max(1, min((8192 + bx - 1) // bx, n // kmin)), (n + kpt - 1) // kpt
+    # (more than 2048 points: below, splits go down to 4 kernels)
     nblk = (m + 255) // 256
-    ns = (16384 + nblk - 1) // nblk
-    return max(1, min(ns, (n + 31) // 32)), n
+    return max(1, min((16384 + nblk - 1) // nblk, (n + 31) // 32)), n
 
 
 def _time_eval(sd, Xd, outd, prec, stream, reps=5):
