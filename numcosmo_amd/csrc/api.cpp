@@ -525,7 +525,10 @@ refresh_bvec (nckde *h)
 }
 
 // points and results of a host-buffer eval up to this size go through the
-// handle's pinned buffer
+// handle's pinned buffer.  Staged against pageable copies: 8 KiB 27 / 39 us, 64
+// KiB 42 / 50, 250 KiB 54 / 56 (d = 4) and 59 / 65 (d = 8); at d = 4 the two meet at 300
+// KiB (512 KiB 76 / 74, 2 MiB 200 / 175), from d = 8 on staging stays 2 to 7 %
+// ahead up to 2 MiB.
 constexpr size_t HOST_STAGE_BYTES = (size_t) 256 << 10;
 
 static int cv_prepare_minimize (nckde *h);
@@ -1499,7 +1502,7 @@ ensure_f32 (nckde *h)
 // nearest in (log2 n, log2 m) within one octave in each, else the default
 // rule: about 8192 blocks in all and at least 8 (DP >= 32) or 256 / DP kernels
 // per split (mixed), about 16384 blocks and at least 32 kernels per split (FP64 and
-// FP32).  Many short splits keep a split's kernel factors in its XCD's L2
+// FP32; shorter ones up to 2048 points, fp64_nsplit).  Many short splits keep a split's kernel factors in its XCD's L2
 // and even out the blocks' finishing times.
 struct SplitTune
 {
