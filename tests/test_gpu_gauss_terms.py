@@ -1,5 +1,5 @@
 """FP64 Gauss terms where a sum against the largest weight constant underflows:
-zero weights, points of other modes, points far out.  Results against the
+zero weights (Student-t too), points of other modes, points far out.  Results against the
 oracle (1e-12, the bar of the FP64 evals), and the kernel's time against that of
 the same call on a plain sample: each pair is visited once wherever it lies."""
 import ctypes as C
@@ -10,7 +10,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def _pair(oracle, kind, d, X, m2lnp=None, local_frac=0.2):
+def _pair(oracle, kind, d, X, local_frac=0.2):
     import numcosmo_amd as na
     sd = (na.StatsDistVKDE if kind == 1 else na.StatsDistKDE).new(na.StatsDistKernelGauss.new(d))
     od = oracle.StatsDist(kind, 0, d, 0.0)
@@ -18,11 +18,7 @@ def _pair(oracle, kind, d, X, m2lnp=None, local_frac=0.2):
         if kind == 1:
             o.set_local_frac(local_frac)
         o.add_obs_array(X)
-        if m2lnp is None:
-            o.prepare()
-        else:
-            o.set_shrink(0.0)
-            o.prepare_interp(m2lnp)
+        o.prepare()
     return sd, od
 
 
@@ -30,14 +26,24 @@ def _err(got, ref):
     return np.max(np.abs(got - ref) / np.maximum(np.abs(ref), 1.0))
 
 
+@pytest.mark.parametrize("nu", [0.0, 3.0, 2.5])
 @pytest.mark.parametrize("kind,d", [(0, 2), (1, 2), (1, 5), (1, 16), (0, 8)])
 @pytest.mark.parametrize("m", [1, 70, 2100])
-def test_zero_weights(oracle, kind, d, m):
+def test_zero_weights(kind, d, m, nu):
     """shrink = 0 leaves the zeros of the active set in the weights (the target is
-    narrower than the sample, so that its outer kernels drop out)."""
+    narrower than the sample, so that its outer kernels drop out; the sample is
+    ordered outwards, so that whole splits have no weight)."""
+    import numcosmo_amd as na
     g = np.random.default_rng(d)
     X = g.normal(size=(400, d))
-    sd, _ = _pair(oracle, kind, d, X, np.minimum(3.0 * np.sum(X * X, 1), 140.0))
+    X = X[np.argsort(np.sum(X * X, 1))]
+    k = na.StatsDistKernelGauss.new(d) if nu == 0.0 else na.StatsDistKernelST.new(d, nu)
+    sd = (na.StatsDistVKDE if kind == 1 else na.StatsDistKDE).new(k)
+    if kind == 1:
+        sd.set_local_frac(0.2)
+    sd.add_obs_array(X)
+    sd.set_shrink(0.0)
+    sd.prepare_interp(np.minimum(3.0 * np.sum(X * X, 1), 140.0))
     assert bool((sd.peek_weights() == 0.0).any())
     P = g.normal(size=(m, d))
     # the density from the device's own weights: two fits of a nearly singular
@@ -48,7 +54,8 @@ def test_zero_weights(oracle, kind, d, m):
     ln = np.array([sd.get_lnnorm(i) for i in live])
     Q = P[-20:]
     z = np.einsum("ikl,pik->pil", Ui, Q[:, None, :] - X[live]) / href
-    t = np.log(w[live]) - 0.5 * np.sum(z * z, 2) - ln
+    chi2 = np.sum(z * z, 2)
+    t = np.log(w[live]) - ln - (0.5 * chi2 if nu == 0.0 else 0.5 * (nu + d) * np.log1p(chi2 / nu))
     mx = t.max(1)
     ref = -2.0 * (mx + np.log(np.sum(np.exp(t - mx[:, None]), 1)))
     # 1e-11: the inverted factors' rounding times chi2
